@@ -11,6 +11,7 @@
 #include <cstring>
 
 #include "device.hpp"
+#include "kernels_f32.hpp"
 
 namespace lrm {
 
@@ -175,41 +176,6 @@ __global__ void k_argmax_rows(const float* x, uint32_t* y, uint32_t rows, uint32
     if (threadIdx.x == 0) y[r] = snan ? 0xFFFFFFFFu : si[0];
 }
 
-// ---------------------------------------------------------------- 12 matmul_bf16w
-// y[i, j] = sum_p fma(x[i, p], widen(w[j, p]), .) from +0 in increasing p: the same chain as CpuRef F32, so the result
-// equals CpuRef's bit for bit and is the same for every m (no split-K, no m-dependent path). A block computes a
-// 16 x 64 tile: thread t owns column t % 64 and rows 4 (t / 64) .. 4 (t / 64) + 3, with k staged 64 at a time.
-constexpr int MM_TM = 16, MM_TN = 64, MM_KS = 64;
-__global__ __launch_bounds__(256) void k_matmul_bf16w(const float* x, const uint16_t* w, float* y, uint32_t m,
-                                                      uint32_t n, uint32_t k) {
-    __shared__ float xs[MM_TM][MM_KS];
-    __shared__ float ws[MM_TN][MM_KS + 1];
-    const uint32_t t = threadIdx.x, col = t % 64u, rg = t / 64u;
-    const uint32_t j0 = blockIdx.x * MM_TN, i0 = blockIdx.y * MM_TM;
-    float acc[4] = {0.f, 0.f, 0.f, 0.f};
-    for (uint32_t p0 = 0; p0 < k; p0 += MM_KS) {
-        uint32_t ks = k - p0 < uint32_t(MM_KS) ? k - p0 : uint32_t(MM_KS);
-        for (uint32_t e = t; e < uint32_t(MM_TM * MM_KS); e += 256u) {
-            uint32_t r = e / MM_KS, p = e % MM_KS;
-            xs[r][p] = (i0 + r < m && p < ks) ? x[size_t(i0 + r) * k + p0 + p] : 0.f;
-        }
-        for (uint32_t e = t; e < uint32_t(MM_TN * MM_KS); e += 256u) {
-            uint32_t c = e / MM_KS, p = e % MM_KS;
-            ws[c][p] = (j0 + c < n && p < ks) ? widen(w[size_t(j0 + c) * k + p0 + p]) : 0.f;
-        }
-        __syncthreads();
-        for (uint32_t p = 0; p < ks; ++p) {
-            float wv = ws[col][p];
-#pragma unroll
-            for (int r = 0; r < 4; ++r) acc[r] = fmaf(xs[rg * 4 + r][p], wv, acc[r]);
-        }
-        __syncthreads();
-    }
-    if (j0 + col < n)
-        for (int r = 0; r < 4; ++r)
-            if (i0 + rg * 4 + r < m) y[size_t(i0 + rg * 4 + r) * n + j0 + col] = acc[r];
-}
-
 // ---------------------------------------------------------------- 13 attention_gqa_causal
 // One 64-thread group per (query row, q head), as the catalog grid. Keys in blocks of 64 anchored at position 0, the
 // causal mask as the loop bound; thread t scores key j0 + t with a sequential fused dot in increasing d (CpuRef's
@@ -332,13 +298,14 @@ static void l_argmax(const PreparedDispatch& pd, void* const* p, hipStream_t s) 
     hipLaunchKernelGGL(k_argmax_rows, phys(pd), dim3(256), 0, s, (const float*)p[0], (uint32_t*)p[1], pd.words[3], pd.words[4]);
 }
 static void l_matmul(const PreparedDispatch& pd, void* const* p, hipStream_t s) {
-    uint32_t m = pd.words[4], n = pd.words[5], k = pd.words[6];
-    dim3 grid((n + MM_TN - 1) / MM_TN, (m + MM_TM - 1) / MM_TM);
-    hipLaunchKernelGGL(k_matmul_bf16w, grid, dim3(256), 0, s, (const float*)p[0], (const uint16_t*)p[1], (float*)p[2], m, n, k);
+    f32k::matmul_bf16w((const float*)p[0], (const uint16_t*)p[1], (float*)p[2], pd.words[4], pd.words[5], pd.words[6], s);
 }
 static void l_attention(const PreparedDispatch& pd, void* const* p, hipStream_t s) {
     uint32_t hd = pd.words[10];
     if (hd > uint32_t(ATT_MAX_HD)) contract_fail("attention_gqa_causal: this device supports head_dim up to %d", ATT_MAX_HD);
+    if (f32k::attention((const float*)p[0], (const float*)p[1], (const float*)p[2], (float*)p[3], pd.words[5], pd.words[6],
+                        pd.words[7], pd.words[8], pd.words[9], hd, f32_of(pd.words[11]), s))
+        return;
     hipLaunchKernelGGL(k_attention_f32, dim3(pd.words[5], pd.words[8]), dim3(64), 0, s, (const float*)p[0],
                        (const float*)p[1], (const float*)p[2], (float*)p[3], pd.words[5], pd.words[6], pd.words[7],
                        pd.words[8], pd.words[9], hd, f32_of(pd.words[11]));
