@@ -17,137 +17,191 @@ namespace f32k {
 using fast::f32x4;
 using fast::lds_barrier;
 using fast::u32x4;
-typedef uint32_t u32x2 __attribute__((ext_vector_type(2)));
+typedef float f32x2 __attribute__((ext_vector_type(2)));
 
 // ---------------------------------------------------------------- matmul_bf16w
-// The operand of step s of a 16x16x4 MFMA holds k = 4 s + g in lane group g = lane / 16. A staged tile therefore keeps
-// each row's k values by group, [row][g][k / 4], so that one LDS read gives a lane four (x, 16 bytes) or four (w, 8
-// bytes) consecutive steps. Row strides 68 and 36 words: the 16 rows of a group start in distinct banks.
-constexpr int KS = 64;            // k per staged tile
-constexpr int XROW = KS + 4;      // words per staged x row
-constexpr int WROW = KS / 2 + 4;  // words per staged w row (bf16 pairs)
+// An output is one chain of k / 4 dependent MFMAs (32 cycles each, 8 per k: what dependent v_fma_f32 take, too), so a
+// wave with one tile must issue its MFMAs back to back. It may issue LDS reads between them for nothing, but every VALU
+// instruction between two dependent MFMAs adds its 4 cycles and every interruption about 8 more (measured: 33 cycles per
+// MFMA alone, 45 with one VALU instruction between, 57 with four; a loop that also widened, staged and addressed took
+// 1170 cycles per 64 k instead of 512). So half of a block's waves only stage: they load x and w (16 bytes per lane, D
+// tiles in flight), widen w and write both to LDS; the others only read operands and multiply. One barrier per tile; the
+// operands of tile t + 1 are read while tile t multiplies and tile t + 2 is stored, NB LDS stages.
+//
+// The operand of step s of a 16x16x4 MFMA holds k = 4 s + g in lane group g = lane / 16, so a staged tile is kept by
+// group, [g][row][k / 4]: one 16-byte LDS read gives a lane four consecutive steps. Rows are KS / 4 + 4 words and a
+// group's plane a multiple of 64: such a read takes 4.2 cycles a wave (rows of KS + 4 words holding all four groups: 8).
 
 // k at or past the end: x = +0 and w = -0, whose product -0 leaves every chain value as it is, -0 included.
 constexpr uint32_t kNegZeroPair = 0x80008000u;
 
-// One block computes a (16 WR TM) x (16 WC TN) tile with WR x WC waves of TM x TN MFMA tiles. D register sets of the
-// next tiles are in flight while the current one multiplies (a step of 64 k takes 0.3 us at one tile per wave, a load
-// from HBM 1-2 us), two LDS stages, one LDS-only barrier per step. The loop runs whole groups of D steps; steps past k
-// multiply the padding.
-// VEC: x and w 16-byte aligned, k a multiple of 8; otherwise element loads.
-template <int WR, int WC, int TM, int TN, int D, bool VEC>
-__global__ __launch_bounds__(256) void k_matmul_mfma(const float* __restrict__ x, const uint16_t* __restrict__ w,
-                                                     float* __restrict__ y, uint32_t m, uint32_t n, uint32_t k) {
-    static_assert(WR * WC == 4, "four waves");
-    constexpr int BM = 16 * WR * TM, BN = 16 * WC * TN;
-    constexpr int XQ = BM * (KS / 4) / 256, WQ = BN * (KS / 8) / 256;  // 16-byte chunks per thread
-    static_assert(XQ >= 1 && WQ >= 1, "whole chunks");
-    __shared__ float xs[2][BM * XROW];
-    __shared__ uint32_t ws[2][BN * WROW];
-    const uint32_t t = threadIdx.x, lane = t & 63u, wv = t >> 6, wr = wv / WC, wc = wv % WC;
+// A block computes a (16 WR TM) x (16 WC TN) tile: WR x WC multiplying waves of TM x TN MFMA tiles, as many staging
+// waves. The loop runs whole groups of D tiles of KS; tiles past k multiply the padding.
+// VEC: x and w 16-byte aligned, k a multiple of 8; otherwise element loads. FULL: k a multiple of D KS, no padding.
+template <int WR, int WC, int TM, int TN, int KS, int D, int NB, bool VEC, bool FULL>
+__global__ __launch_bounds__(128 * WR * WC) void k_matmul_mfma(const float* __restrict__ x,
+                                                               const uint16_t* __restrict__ w, float* __restrict__ y,
+                                                               uint32_t m, uint32_t n, uint32_t k) {
+    constexpr int BM = 16 * WR * TM, BN = 16 * WC * TN, NT = 64 * WR * WC, STEPS = KS / 4, ROW = STEPS + 4;
+    constexpr int XR = NT / (KS / 4), WRW = NT / (KS / 8);  // rows staged per pass
+    constexpr int XQ = BM / XR, WQ = BN / WRW;              // 16-byte chunks per staging thread
+    static_assert(XQ >= 1 && WQ >= 1 && BM % XR == 0 && BN % WRW == 0, "whole chunks");
+    static_assert(D % NB == 0 && NB >= 3 && D % 2 == 0, "stages and operand sets of the unrolled loop");
+    static_assert(KS == 64, "chunk maps");
+    __shared__ float xs[NB][4 * BM * ROW];
+    __shared__ float ws[NB][4 * BN * ROW];
     const uint32_t i0 = blockIdx.y * BM, j0 = blockIdx.x * BN;
-    // chunk q of this thread: x row xr(q), k 4 xc ..; a wave's four rows are 4 apart (distinct banks when stored)
-    const uint32_t xc = t & 15u, xr0 = ((t >> 4) & 3u) * 4u + (t >> 6);
-    const uint32_t wcx = t & 7u, wr0 = t >> 3;
-    u32x4 xreg[D][XQ], wreg[D][WQ];
-
-    auto load = [&](int d, uint32_t k0) {
+    if (threadIdx.x >= NT) {
+        const uint32_t t = threadIdx.x - NT;
+        // chunk q of this thread: x row xr0 + XR q, k 4 xc ..; w row wr0 + WRW q, k 8 wcx ..; the rows a store touches
+        // at once lie four apart (distinct banks)
+        const uint32_t xc = t & (KS / 4 - 1), wcx = t & (KS / 8 - 1);
+        const uint32_t xr0 = ((t >> 4) & 3u) * (XR / 4) + (t >> 6);
+        const uint32_t wr0 = NT >= 128
+                                 ? ((t >> 3) & 3u) * 4u + ((t >> 5) & 1u) + ((t >> 6) & 1u) * 2u + (t >> 7) * 16u
+                                 : t / (KS / 8);
+        u32x4 xreg[D][XQ], wreg[D][WQ];
+        // FULL: buffer loads, the k offset in a scalar register. A VALU instruction of this wave also delays the
+        // multiplying wave of its SIMD, and 64-bit addresses took most of them.
+        const uint32_t xrows = m - i0 < uint32_t(BM) ? m - i0 : uint32_t(BM);
+        const uint32_t wrows = n - j0 < uint32_t(BN) ? n - j0 : uint32_t(BN);
+        const auto xrsrc = __builtin_amdgcn_make_buffer_rsrc(const_cast<float*>(x + size_t(i0) * k), (short)0,
+                                                             int(xrows * k * 4u), 0x00020000);
+        const auto wrsrc = __builtin_amdgcn_make_buffer_rsrc(const_cast<uint16_t*>(w + size_t(j0) * k), (short)0,
+                                                             int(wrows * k * 2u), 0x00020000);
+        uint32_t xo[XQ], wo[WQ];
 #pragma unroll
-        for (int q = 0; q < XQ; ++q) {
-            uint32_t row = i0 + xr0 + 16u * q;
-            row = row < m ? row : m - 1u;
-            const uint32_t kk = k0 + 4u * xc;
-            if constexpr (VEC) {
-                xreg[d][q] = *reinterpret_cast<const u32x4*>(x + size_t(row) * k + (kk < k ? kk : 0u));
-            } else {
+        for (int q = 0; q < XQ; ++q) xo[q] = (xr0 + XR * q < xrows ? xr0 + XR * q : xrows - 1u) * k * 4u + 16u * xc;
 #pragma unroll
-                for (uint32_t e = 0; e < 4; ++e)
-                    xreg[d][q][e] = __float_as_uint(x[size_t(row) * k + (kk + e < k ? kk + e : 0u)]);
+        for (int q = 0; q < WQ; ++q) wo[q] = (wr0 + WRW * q < wrows ? wr0 + WRW * q : wrows - 1u) * k * 2u + 16u * wcx;
+        auto load = [&](int d, uint32_t k0) {
+            if constexpr (FULL) {
+                const uint32_t ks = k0 < k ? k0 : k - KS;  // (a tile past the last: the last, never multiplied)
+#pragma unroll
+                for (int q = 0; q < XQ; ++q) xreg[d][q] = __builtin_amdgcn_raw_buffer_load_b128(xrsrc, xo[q], ks * 4u, 0);
+#pragma unroll
+                for (int q = 0; q < WQ; ++q) wreg[d][q] = __builtin_amdgcn_raw_buffer_load_b128(wrsrc, wo[q], ks * 2u, 0);
+                __builtin_amdgcn_sched_barrier(0);
+                return;
             }
-        }
 #pragma unroll
-        for (int q = 0; q < WQ; ++q) {
-            uint32_t col = j0 + wr0 + 32u * q;
-            col = col < n ? col : n - 1u;
-            const uint32_t kk = k0 + 8u * wcx;
-            if constexpr (VEC) {
-                wreg[d][q] = *reinterpret_cast<const u32x4*>(w + size_t(col) * k + (kk < k ? kk : 0u));
-            } else {
+            for (int q = 0; q < XQ; ++q) {
+                uint32_t row = i0 + xr0 + XR * q;
+                row = row < m ? row : m - 1u;
+                const uint32_t kk = k0 + 4u * xc;
+                if constexpr (VEC) {
+                    xreg[d][q] = *reinterpret_cast<const u32x4*>(x + size_t(row) * k + (kk < k ? kk : 0u));
+                } else {
 #pragma unroll
-                for (uint32_t e = 0; e < 4; ++e) {
-                    const uint32_t a = kk + 2u * e, b = a + 1u;
-                    const uint32_t lo = w[size_t(col) * k + (a < k ? a : 0u)], hi = w[size_t(col) * k + (b < k ? b : 0u)];
-                    wreg[d][q][e] = (a < k ? lo : 0x8000u) | (b < k ? hi << 16 : 0x80000000u);
+                    for (uint32_t e = 0; e < 4; ++e)
+                        xreg[d][q][e] = __float_as_uint(x[size_t(row) * k + (kk + e < k ? kk + e : 0u)]);
                 }
             }
-        }
-    };
-    auto store = [&](int d, int buf, uint32_t k0) {
 #pragma unroll
-        for (int q = 0; q < XQ; ++q) {
-            const uint32_t kk = k0 + 4u * xc;
-            float* p = &xs[buf][(xr0 + 16u * q) * XROW + xc];
+            for (int q = 0; q < WQ; ++q) {
+                uint32_t col = j0 + wr0 + WRW * q;
+                col = col < n ? col : n - 1u;
+                const uint32_t kk = k0 + 8u * wcx;
+                if constexpr (VEC) {
+                    wreg[d][q] = *reinterpret_cast<const u32x4*>(w + size_t(col) * k + (kk < k ? kk : 0u));
+                } else {
 #pragma unroll
-            for (uint32_t g = 0; g < 4; ++g) {
-                const bool in = VEC ? kk < k : kk + g < k;
-                p[g * (KS / 4)] = in ? __uint_as_float(xreg[d][q][g]) : 0.f;
+                    for (uint32_t e = 0; e < 4; ++e) {
+                        const uint32_t a = kk + 2u * e, b = a + 1u;
+                        const uint32_t lo = w[size_t(col) * k + (a < k ? a : 0u)],
+                                       hi = w[size_t(col) * k + (b < k ? b : 0u)];
+                        wreg[d][q][e] = (a < k ? lo : 0x8000u) | (b < k ? hi << 16 : 0x80000000u);
+                    }
+                }
             }
-        }
+            __builtin_amdgcn_sched_barrier(0);
+        };
+        auto store = [&](int d, uint32_t k0) {  // set d's tile (at k0) to LDS stage d % NB
 #pragma unroll
-        for (int q = 0; q < WQ; ++q) {
-            u32x4 v = wreg[d][q];
-            if (VEC && k0 + 8u * wcx >= k) v = u32x4{kNegZeroPair, kNegZeroPair, kNegZeroPair, kNegZeroPair};
-            uint32_t* p = &ws[buf][(wr0 + 32u * q) * WROW + wcx];
-            p[0] = (v[0] & 0xFFFFu) | (v[2] << 16);
-            p[8] = (v[0] >> 16) | (v[2] & 0xFFFF0000u);
-            p[16] = (v[1] & 0xFFFFu) | (v[3] << 16);
-            p[24] = (v[1] >> 16) | (v[3] & 0xFFFF0000u);
-        }
-    };
-
-    f32x4 acc[TM][TN];
+            for (int q = 0; q < XQ; ++q) {
+                const uint32_t kk = k0 + 4u * xc;
+                float* p = &xs[d % NB][(xr0 + XR * q) * ROW + xc];
+#pragma unroll
+                for (uint32_t g = 0; g < 4; ++g) {
+                    const bool in = FULL || (VEC ? kk < k : kk + g < k);
+                    p[g * BM * ROW] = in ? __uint_as_float(xreg[d][q][g]) : 0.f;
+                }
+            }
+#pragma unroll
+            for (int q = 0; q < WQ; ++q) {
+                u32x4 v = wreg[d][q];
+                if (VEC && !FULL && k0 + 8u * wcx >= k) v = u32x4{kNegZeroPair, kNegZeroPair, kNegZeroPair, kNegZeroPair};
+                float* p = &ws[d % NB][(wr0 + WRW * q) * ROW + 2 * wcx];
+#pragma unroll
+                for (int g = 0; g < 4; ++g) {  // k 8 wcx + g and + 4 + g
+                    const uint32_t a = v[g >> 1], b = v[2 + (g >> 1)];
+                    f32x2 pair;
+                    pair[0] = __uint_as_float((g & 1) ? a & 0xFFFF0000u : a << 16);
+                    pair[1] = __uint_as_float((g & 1) ? b & 0xFFFF0000u : b << 16);
+                    *reinterpret_cast<f32x2*>(p + g * BN * ROW) = pair;
+                }
+            }
+            __builtin_amdgcn_sched_barrier(0);
+        };
+#pragma unroll
+        for (int d = 0; d < D; ++d) load(d, uint32_t(d) * KS);
+        store(0, 0);
+        store(1, KS);
+        lds_barrier();
+        uint32_t k0 = 0;
+        do {  // (at least once: a loop that may not run lets the compiler sink the first loads past the barrier above)
+#pragma unroll
+            for (int d = 0; d < D; ++d) {
+                load(d, k0 + uint32_t(d + D) * KS);  // this set's tile is in LDS
+                store((d + 2) % D, k0 + uint32_t(d + 2) * KS);
+                lds_barrier();
+            }
+            k0 += D * KS;
+        } while (k0 < k);
+        return;
+    }
+    const uint32_t lane = threadIdx.x & 63u, wv = threadIdx.x >> 6, wr = wv / WC, wc = wv % WC;
+    const uint32_t r16 = lane & 15u, grp = lane >> 4;
+    const uint32_t xoff = (grp * BM + wr * TM * 16u + r16) * ROW, woff = (grp * BN + wc * TN * 16u + r16) * ROW;
+    f32x4 acc[TM][TN], av[2][TM][STEPS / 4], bv[2][TN][STEPS / 4];
 #pragma unroll
     for (int a = 0; a < TM; ++a)
 #pragma unroll
         for (int b = 0; b < TN; ++b) acc[a][b] = f32x4{0.f, 0.f, 0.f, 0.f};
-    const uint32_t r16 = lane & 15u, grp = lane >> 4;
-    auto compute = [&](int buf) {
-        const float* xb = &xs[buf][(wr * TM * 16u + r16) * XROW + grp * (KS / 4)];
-        const uint32_t* wb = &ws[buf][(wc * TN * 16u + r16) * WROW + grp * (KS / 8)];
+    auto read = [&](int set, int d) {
 #pragma unroll
-        for (int q = 0; q < KS / 16; ++q) {
-            f32x4 av[TM];
-            u32x2 bv[TN];
+        for (int q = 0; q < STEPS / 4; ++q) {
 #pragma unroll
-            for (int a = 0; a < TM; ++a) av[a] = *reinterpret_cast<const f32x4*>(xb + a * 16 * XROW + 4 * q);
+            for (int a = 0; a < TM; ++a)
+                av[set][a][q] = *reinterpret_cast<const f32x4*>(&xs[d % NB][xoff + a * 16 * ROW + 4 * q]);
 #pragma unroll
-            for (int b = 0; b < TN; ++b) bv[b] = *reinterpret_cast<const u32x2*>(wb + b * 16 * WROW + 2 * q);
-#pragma unroll
-            for (int i = 0; i < 4; ++i)
-#pragma unroll
-                for (int a = 0; a < TM; ++a)
-#pragma unroll
-                    for (int b = 0; b < TN; ++b) {
-                        const uint32_t h = bv[b][i >> 1];
-                        acc[a][b] = __builtin_amdgcn_mfma_f32_16x16x4f32(
-                            av[a][i], __uint_as_float((i & 1) ? h & 0xFFFF0000u : h << 16), acc[a][b], 0, 0, 0);
-                    }
+            for (int b = 0; b < TN; ++b)
+                bv[set][b][q] = *reinterpret_cast<const f32x4*>(&ws[d % NB][woff + b * 16 * ROW + 4 * q]);
         }
+        __builtin_amdgcn_sched_barrier(0);
     };
-
-#pragma unroll
-    for (int d = 0; d < D; ++d) load(d, uint32_t(d) * KS);
-    store(0, 0, 0);
     lds_barrier();
-    for (uint32_t k0 = 0; k0 < k; k0 += D * KS) {
+    read(0, 0);
+    uint32_t k0 = 0;
+    do {
 #pragma unroll
         for (int d = 0; d < D; ++d) {
-            load(d, k0 + uint32_t(d + D) * KS);  // this set's tile is in LDS
-            compute(d & 1);
-            store((d + 1) % D, (d + 1) & 1, k0 + uint32_t(d + 1) * KS);
+            read((d + 1) & 1, d + 1);
+#pragma unroll
+            for (int q = 0; q < STEPS / 4; ++q)
+#pragma unroll
+                for (int i = 0; i < 4; ++i)
+#pragma unroll
+                    for (int a = 0; a < TM; ++a)
+#pragma unroll
+                        for (int b = 0; b < TN; ++b)
+                            acc[a][b] = __builtin_amdgcn_mfma_f32_16x16x4f32(av[d & 1][a][q][i], bv[d & 1][b][q][i],
+                                                                             acc[a][b], 0, 0, 0);
+            __builtin_amdgcn_sched_barrier(0);
             lds_barrier();
         }
-    }
+        k0 += D * KS;
+    } while (k0 < k);
 #pragma unroll
     for (int a = 0; a < TM; ++a)
 #pragma unroll
@@ -161,124 +215,36 @@ __global__ __launch_bounds__(256) void k_matmul_mfma(const float* __restrict__ x
         }
 }
 
-// One or two rows of x (a decode step): an output is one dependent chain, so its k fused adds bound the kernel (5-6
-// cycles each: the add and its share of the LDS reads), not the weights. A block owns 32 columns: wave 4 runs the chains
-// (lane = column + 32 row), waves 0-3 load the weights (16 bytes per lane, D tiles of 128 k in flight), widen them to
-// float32 into LDS, two stages, one barrier per tile. 32 columns and not 64: the weights of one block come through one
-// CU, and at 64 columns that stream is slower than the chain.
-constexpr int ROW_C = 32, ROW_KT = 128, ROW_STRIDE = ROW_KT + 4, ROW_D = 4;
-__global__ __launch_bounds__(320) void k_matmul_row(const float* __restrict__ x, const uint16_t* __restrict__ w,
-                                                    float* __restrict__ y, uint32_t m, uint32_t n, uint32_t k) {
-    __shared__ float ws[2][ROW_C * ROW_STRIDE];
-    __shared__ float xs[2][2][ROW_KT];
-    const uint32_t t = threadIdx.x, j0 = blockIdx.x * ROW_C;
-    const uint32_t tiles = (k + ROW_KT - 1) / ROW_KT, rounds = (tiles + ROW_D - 1) / ROW_D;
-    if (t < 256) {
-        const uint32_t c = t & 15u, col0 = t >> 4;  // chunk: 8 k of column col0 (and col0 + 16)
-        const uint32_t xrow = (t >> 5) < m ? t >> 5 : m - 1u, xc = t & 31u;
-        u32x4 wreg[ROW_D][2];
-        f32x4 xreg[ROW_D];
-        auto load = [&](int d, uint32_t k0) {
-#pragma unroll
-            for (int q = 0; q < 2; ++q) {
-                uint32_t col = j0 + col0 + 16u * q;
-                col = col < n ? col : n - 1u;
-                const uint32_t kk = k0 + 8u * c;
-                wreg[d][q] = *reinterpret_cast<const u32x4*>(w + size_t(col) * k + (kk < k ? kk : 0u));
-            }
-            if (t < 64) {
-                const uint32_t kk = k0 + 4u * xc;
-                xreg[d] = *reinterpret_cast<const f32x4*>(x + size_t(xrow) * k + (kk < k ? kk : 0u));
-            }
-        };
-        auto store = [&](int d, int buf, uint32_t k0) {
-            const bool in = k0 + 8u * c < k;
-#pragma unroll
-            for (int q = 0; q < 2; ++q) {
-                u32x4 v = wreg[d][q];
-                if (!in) v = u32x4{kNegZeroPair, kNegZeroPair, kNegZeroPair, kNegZeroPair};
-                float* p = &ws[buf][(col0 + 16u * q) * ROW_STRIDE + 8u * c];
-                f32x4 a, b;
-#pragma unroll
-                for (int e = 0; e < 2; ++e) {
-                    a[2 * e] = __uint_as_float(v[e] << 16);
-                    a[2 * e + 1] = __uint_as_float(v[e] & 0xFFFF0000u);
-                    b[2 * e] = __uint_as_float(v[e + 2] << 16);
-                    b[2 * e + 1] = __uint_as_float(v[e + 2] & 0xFFFF0000u);
-                }
-                *reinterpret_cast<f32x4*>(p) = a;
-                *reinterpret_cast<f32x4*>(p + 4) = b;
-            }
-            if (t < 64) {
-                f32x4 v = xreg[d];
-                if (k0 + 4u * xc >= k) v = f32x4{0.f, 0.f, 0.f, 0.f};
-                *reinterpret_cast<f32x4*>(&xs[buf][t >> 5][4u * xc]) = v;
-            }
-        };
-#pragma unroll
-        for (int d = 0; d < ROW_D; ++d) load(d, uint32_t(d) * ROW_KT);
-        store(0, 0, 0);
-        lds_barrier();
-        for (uint32_t r = 0; r < rounds; ++r) {
-            const uint32_t k0 = r * ROW_D * ROW_KT;
-#pragma unroll
-            for (int d = 0; d < ROW_D; ++d) {
-                load(d, k0 + uint32_t(d + ROW_D) * ROW_KT);
-                store((d + 1) % ROW_D, (d + 1) & 1, k0 + uint32_t(d + 1) * ROW_KT);
-                lds_barrier();
-            }
-        }
-    } else {
-        const uint32_t lane = t - 256u, col = lane & 31u, row = lane >> 5;
-        float acc = 0.f;
-        lds_barrier();
-        for (uint32_t r = 0; r < rounds; ++r) {
-#pragma unroll
-            for (int d = 0; d < ROW_D; ++d) {
-                const float* wp = &ws[d & 1][col * ROW_STRIDE];
-                const float* xp = xs[d & 1][row];
-#pragma unroll
-                for (int q = 0; q < ROW_KT / 4; ++q) {
-                    const f32x4 a = *reinterpret_cast<const f32x4*>(xp + 4 * q);
-                    const f32x4 b = *reinterpret_cast<const f32x4*>(wp + 4 * q);
-#pragma unroll
-                    for (int e = 0; e < 4; ++e) acc = fmaf(a[e], b[e], acc);
-                }
-                lds_barrier();
-            }
-        }
-        if (row < m && j0 + col < n) y[size_t(row) * n + j0 + col] = acc;
-    }
-}
-
 static bool aligned16(const void* p) { return (reinterpret_cast<uintptr_t>(p) & 15u) == 0; }
 
-template <int WR, int WC, int TM, int TN, int D>
+template <int WR, int WC, int TM, int TN, int KS, int D, int NB>
 static void launch_mfma(bool vec, const float* x, const uint16_t* w, float* y, uint32_t m, uint32_t n, uint32_t k,
                         hipStream_t s) {
     constexpr uint32_t BM = 16 * WR * TM, BN = 16 * WC * TN;
-    const dim3 grid((n + BN - 1) / BN, (m + BM - 1) / BM);
-    if (vec)
-        hipLaunchKernelGGL((k_matmul_mfma<WR, WC, TM, TN, D, true>), grid, dim3(256), 0, s, x, w, y, m, n, k);
+    const dim3 grid((n + BN - 1) / BN, (m + BM - 1) / BM), block(128 * WR * WC);
+    if (vec && k % (D * KS) == 0 && uint64_t(k) * (BM > BN / 2 ? BM : BN / 2) * 4 < (1ull << 31))
+        hipLaunchKernelGGL((k_matmul_mfma<WR, WC, TM, TN, KS, D, NB, true, true>), grid, block, 0, s, x, w, y, m, n, k);
+    else if (vec)
+        hipLaunchKernelGGL((k_matmul_mfma<WR, WC, TM, TN, KS, D, NB, true, false>), grid, block, 0, s, x, w, y, m, n, k);
     else
-        hipLaunchKernelGGL((k_matmul_mfma<WR, WC, TM, TN, D, false>), grid, dim3(256), 0, s, x, w, y, m, n, k);
+        hipLaunchKernelGGL((k_matmul_mfma<WR, WC, TM, TN, KS, D, NB, false, false>), grid, block, 0, s, x, w, y, m, n, k);
 }
 
 void matmul_bf16w(const float* x, const uint16_t* w, float* y, uint32_t m, uint32_t n, uint32_t k, hipStream_t s) {
     const bool vec = k % 8 == 0 && aligned16(x) && aligned16(w);
-    if (m <= 2 && vec) {
-        hipLaunchKernelGGL(k_matmul_row, dim3((n + ROW_C - 1) / ROW_C), dim3(320), 0, s, x, w, y, m, n, k);
-        return;
-    }
-    // 64 x 64 tiles when they give every CU two blocks, else 32 x 32 (four times the blocks), or 16 x 64 for the rows
-    // of one MFMA tile
-    const uint64_t big = uint64_t((m + 63) / 64) * ((n + 63) / 64);
-    if (m <= 16)
-        launch_mfma<1, 4, 1, 1, 4>(vec, x, w, y, m, n, k, s);
-    else if (big >= 512)
-        launch_mfma<2, 2, 2, 2, 2>(vec, x, w, y, m, n, k, s);
+    // Up to 16 rows one MFMA tile per block: an output is one chain however many columns a block has, and two waves find
+    // SIMDs of their own (1 x 1024 x 1024: 5.8 us; 32-column blocks 6.0); past 16,384 columns, where the weights' stream
+    // counts, 32 columns (1 x 151,936 x 1024: 79.7 us against 84.1). Above: 32 x 32 tiles (150 x 3072 x 1024: 14.7 us;
+    // 64 x 64 22.1), 64 x 64 from 200 of those tiles on (300 x 3072 x 1024, 240 tiles: 23.2 against 26.3; 2048 x 3072 x
+    // 1024: 126 against 139, 102 TFLOP/s; 300 x 2048 x 1024, 160 tiles: 22.2 against 20.5).
+    if (m <= 16 && n <= 16384)
+        launch_mfma<1, 1, 1, 1, 64, 4, 4>(vec, x, w, y, m, n, k, s);
+    else if (m <= 16)
+        launch_mfma<1, 2, 1, 1, 64, 8, 4>(vec, x, w, y, m, n, k, s);
+    else if (uint64_t((m + 63) / 64) * ((n + 63) / 64) >= 200)
+        launch_mfma<2, 2, 2, 2, 64, 4, 4>(vec, x, w, y, m, n, k, s);
     else
-        launch_mfma<2, 2, 1, 1, 4>(vec, x, w, y, m, n, k, s);
+        launch_mfma<2, 2, 1, 1, 64, 8, 4>(vec, x, w, y, m, n, k, s);
 }
 
 // ---------------------------------------------------------------- attention_gqa_causal
@@ -336,36 +302,67 @@ __global__ __launch_bounds__(W == 1 ? 256 : 64 * W) void k_attention_mfma(
     const size_t qoff = (size_t(q_row0 + row) * qh + head) * HD;
 
     float qf[U][4];
-#pragma unroll
-    for (int u = 0; u < U; ++u) {
-        const f32x4 v = *reinterpret_cast<const f32x4*>(q + qoff + 16 * u + 4u * grp);
-#pragma unroll
-        for (int i = 0; i < 4; ++i) qf[u][i] = v[i];
-        transpose4(qf[u]);
-    }
-
-    // scores of block b: s[t][r] = key 64 b + 16 t + 4 grp + r (times scale); returns the block's maximum over this
-    // column's keys (-inf for none)
-    auto score = [&](uint32_t b, f32x4 (&s)[4]) {
-        float mx = -INFINITY;
+    // A block's K and V come in whole: all loads in flight at once (the compiler, left alone, keeps a few), V's while
+    // the scores' maxima meet, the next block's K while the values are combined.
+    auto load_k = [&](uint32_t b, f32x4 (&kr)[U][4]) {
+        const float* p[4];
 #pragma unroll
         for (int t = 0; t < 4; ++t) {
             const uint32_t j = b * 64u + 16u * t + col;
-            const float* kr = kb + size_t(j < max_keys ? j : max_keys - 1u) * kv_stride;
-            f32x4 a = {0.f, 0.f, 0.f, 0.f};
+            p[t] = kb + size_t(j < max_keys ? j : max_keys - 1u) * kv_stride;
+        }
 #pragma unroll
-            for (int u = 0; u < U; ++u) {
-                const f32x4 kv = *reinterpret_cast<const f32x4*>(kr + 16 * u);
-                float kf[4] = {kv[0], kv[1], kv[2], kv[3]};
-                transpose4(kf);
+        for (int u = 0; u < U; ++u)
 #pragma unroll
-                for (int i = 0; i < 4; ++i) a = __builtin_amdgcn_mfma_f32_16x16x4f32(kf[i], qf[u][i], a, 0, 0, 0);
+            for (int t = 0; t < 4; ++t) kr[u][t] = *reinterpret_cast<const f32x4*>(p[t] + 16 * u);
+        __builtin_amdgcn_sched_barrier(0);
+    };
+    // E values of each tile group c at step st: key 64 b + 4 st + grp (a key past the tile's last: its last)
+    auto load_v = [&](uint32_t b, float (&vr)[16][NC][E]) {
+#pragma unroll
+        for (int st = 0; st < 16; ++st) {
+            const uint32_t j = b * 64u + 4u * st + grp;
+            const float* p = vb + size_t(j < max_keys ? j : max_keys - 1u) * kv_stride;
+#pragma unroll
+            for (int c = 0; c < NC; ++c) {
+                if constexpr (E == 4) {
+                    const f32x4 x = *reinterpret_cast<const f32x4*>(p + 64 * c);
+#pragma unroll
+                    for (int e = 0; e < 4; ++e) vr[st][c][e] = x[e];
+                } else {
+                    vr[st][c][0] = p[16 * c];
+                }
             }
+        }
+        __builtin_amdgcn_sched_barrier(0);
+    };
+    // scores of block b: s[t][r] = key 64 b + 16 t + 4 grp + r (times scale); returns the block's maximum over this
+    // column's keys (-inf for none)
+    auto score = [&](uint32_t b, const f32x4 (&kr)[U][4], f32x4 (&s)[4]) {
+        float mx = -INFINITY;
+#pragma unroll
+        for (int t = 0; t < 4; ++t) s[t] = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+            float kf[4][4];
+#pragma unroll
+            for (int t = 0; t < 4; ++t) {
+#pragma unroll
+                for (int i = 0; i < 4; ++i) kf[t][i] = kr[u][t][i];
+                transpose4(kf[t]);
+            }
+#pragma unroll
+            for (int i = 0; i < 4; ++i)
+#pragma unroll
+                for (int t = 0; t < 4; ++t) s[t] = __builtin_amdgcn_mfma_f32_16x16x4f32(kf[t][i], qf[u][i], s[t], 0, 0, 0);
+        }
+#pragma unroll
+        for (int t = 0; t < 4; ++t) {
 #pragma unroll
             for (int r = 0; r < 4; ++r) {
                 // a key past the column's own scores -inf: weight 0 (or NaN where every score is -inf or NaN, and the
                 // reference's weights are NaN too)
-                s[t][r] = b * 64u + 16u * t + 4u * grp + r < keys ? a[r] * scale : -INFINITY;
+                s[t][r] = b * 64u + 16u * t + 4u * grp + r < keys ? s[t][r] * scale : -INFINITY;
                 mx = fmaxf(mx, s[t][r]);
             }
         }
@@ -374,45 +371,30 @@ __global__ __launch_bounds__(W == 1 ? 256 : 64 * W) void k_attention_mfma(
 
     // the block's values and sum against the maximum mn: acc (register (c, e, r) = dimension 16 E c + E (4 grp + r) + e
     // of this column), bs the sum of the weights
-    auto values = [&](uint32_t b, const f32x4 (&s)[4], float mn, f32x4 (&acc)[NC][E], float& bs) {
+    auto values = [&](uint32_t b, const f32x4 (&s)[4], float mn, const float (&vr)[16][NC][E], f32x4 (&acc)[NC][E],
+                      float& bs) {
         float pf[4][4];
 #pragma unroll
         for (int t = 0; t < 4; ++t) {
 #pragma unroll
-            for (int r = 0; r < 4; ++r)
-                pf[t][r] = expf(s[t][r] - mn);
+            for (int r = 0; r < 4; ++r) pf[t][r] = expf(s[t][r] - mn);
             transpose4(pf[t]);
         }
         f32x4 sum = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
         for (int st = 0; st < 16; ++st) sum = __builtin_amdgcn_mfma_f32_16x16x4f32(1.f, pf[st >> 2][st & 3], sum, 0, 0, 0);
         bs = sum[0];
-        // this lane's E values of tile group c at step st (a key past the tile's last: its last)
-        auto value = [&](int st, int c, float (&vv)[E]) {
-            const uint32_t j = b * 64u + 4u * st + grp;
-            const float* vr = vb + size_t(j < max_keys ? j : max_keys - 1u) * kv_stride + 16 * E * c;
-            if constexpr (E == 4) {
-                const f32x4 l = *reinterpret_cast<const f32x4*>(vr);
-#pragma unroll
-                for (int e = 0; e < 4; ++e) vv[e] = l[e];
-            } else {
-                vv[0] = vr[0];
-            }
-        };
         // A key past a column's own has weight 0, which leaves the chain as it is only while its value is finite: where
         // a block with such keys holds an infinity or a NaN, each column runs alone with those values zeroed.
         bool odd = false;
         if (b * 64u + 64u > first_keys) {
             uint32_t bad = 0;
-#pragma unroll 4
+#pragma unroll
             for (int st = 0; st < 16; ++st)
 #pragma unroll
-                for (int c = 0; c < NC; ++c) {
-                    float vv[E];
-                    value(st, c, vv);
+                for (int c = 0; c < NC; ++c)
 #pragma unroll
-                    for (int e = 0; e < E; ++e) bad |= uint32_t(!finite(vv[e]));
-                }
+                    for (int e = 0; e < E; ++e) bad |= uint32_t(!finite(vr[st][c][e]));
             odd = __ballot(bad != 0u) != 0;
         }
 #pragma unroll
@@ -423,13 +405,11 @@ __global__ __launch_bounds__(W == 1 ? 256 : 64 * W) void k_attention_mfma(
 #pragma unroll
             for (int st = 0; st < 16; ++st)
 #pragma unroll
-                for (int c = 0; c < NC; ++c) {
-                    float vv[E];
-                    value(st, c, vv);
+                for (int c = 0; c < NC; ++c)
 #pragma unroll
                     for (int e = 0; e < E; ++e)
-                        acc[c][e] = __builtin_amdgcn_mfma_f32_16x16x4f32(vv[e], pf[st >> 2][st & 3], acc[c][e], 0, 0, 0);
-                }
+                        acc[c][e] =
+                            __builtin_amdgcn_mfma_f32_16x16x4f32(vr[st][c][e], pf[st >> 2][st & 3], acc[c][e], 0, 0, 0);
             return;
         }
 #pragma unroll 1
@@ -442,14 +422,11 @@ __global__ __launch_bounds__(W == 1 ? 256 : 64 * W) void k_attention_mfma(
 #pragma unroll
                 for (int e = 0; e < E; ++e) a[e] = f32x4{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-                for (int st = 0; st < 16; ++st) {
-                    float vv[E];
-                    value(st, c, vv);
+                for (int st = 0; st < 16; ++st)
 #pragma unroll
                     for (int e = 0; e < E; ++e)
-                        a[e] = __builtin_amdgcn_mfma_f32_16x16x4f32(4 * st < own ? vv[e] : 0.f, pf[st >> 2][st & 3], a[e], 0,
-                                                                    0, 0);
-                }
+                        a[e] = __builtin_amdgcn_mfma_f32_16x16x4f32(4 * st < own ? vr[st][c][e] : 0.f,
+                                                                    pf[st >> 2][st & 3], a[e], 0, 0, 0);
 #pragma unroll
                 for (int e = 0; e < E; ++e)
 #pragma unroll
@@ -458,6 +435,15 @@ __global__ __launch_bounds__(W == 1 ? 256 : 64 * W) void k_attention_mfma(
         }
     };
 
+    f32x4 k0[U][4];
+    load_k(W == 1 ? 0u : wv, k0);  // (ahead of q)
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+        const f32x4 v = *reinterpret_cast<const f32x4*>(q + qoff + 16 * u + 4u * grp);
+#pragma unroll
+        for (int i = 0; i < 4; ++i) qf[u][i] = v[i];
+        transpose4(qf[u]);
+    }
     float m = 0.f, l = 0.f;
     if constexpr (W == 1) {
         f32x4 o[NC][E];
@@ -467,12 +453,15 @@ __global__ __launch_bounds__(W == 1 ? 256 : 64 * W) void k_attention_mfma(
             for (int e = 0; e < E; ++e) o[c][e] = f32x4{0.f, 0.f, 0.f, 0.f};
         for (uint32_t b = 0; b < nblocks; ++b) {
             f32x4 s[4], acc[NC][E];
-            const float bmax = score(b, s);
+            float vr[16][NC][E];
+            const float bmax = score(b, k0, s);
+            load_v(b, vr);
             const bool active = b * 64u < keys;  // a column without keys in this block keeps its state
             if (b == 0) m = bmax;
             const float mn = fmaxf(m, bmax), alpha = expf(m - mn);
             float bs;
-            values(b, s, mn, acc, bs);
+            values(b, s, mn, vr, acc, bs);
+            load_k(b + 1, k0);
             if (active) {
                 m = mn;
                 l = fmaf(l, alpha, bs);
@@ -506,28 +495,29 @@ __global__ __launch_bounds__(W == 1 ? 256 : 64 * W) void k_attention_mfma(
         for (uint32_t b0 = 0; b0 < nblocks; b0 += W) {
             const uint32_t b = b0 + wv;
             f32x4 s[4];
+            float vr[16][NC][E];
             if (b < nblocks) {
-                const float bmax = score(b, s);
+                const float bmax = score(b, k0, s);
                 if (grp == 0) sm[wv][col] = bmax;
             }
+            load_v(b, vr);  // (past the last block: its last row; a load under a condition would keep two sets alive)
             lds_barrier();
-            float mn = 0.f, alpha[W];
+            float mn = 0.f, alpha[W], bm[W];
+#pragma unroll
+            for (int i = 0; i < W; ++i) bm[i] = sm[i][col];
+            m = b0 == 0 ? bm[0] : m;
 #pragma unroll
             for (int i = 0; i < W; ++i) {
-                alpha[i] = 1.f;
-                if ((b0 + i) * 64u < keys) {
-                    const float bm = sm[i][col];
-                    if (b0 + i == 0) m = bm;
-                    const float nx = fmaxf(m, bm);
-                    alpha[i] = expf(m - nx);
-                    m = nx;
-                }
+                const bool active = (b0 + i) * 64u < keys;  // a column without keys in this block keeps its state
+                const float nx = fmaxf(m, bm[i]), al = expf(m - nx);
+                alpha[i] = active ? al : 1.f;
+                m = active ? nx : m;
                 if (uint32_t(i) == wv) mn = m;
             }
             if (b < nblocks) {
                 f32x4 acc[NC][E];
                 float bs;
-                values(b, s, mn, acc, bs);
+                values(b, s, mn, vr, acc, bs);
                 if (grp == 0) ssum[wv][col] = bs;
 #pragma unroll
                 for (int c = 0; c < NC; ++c)
@@ -536,16 +526,21 @@ __global__ __launch_bounds__(W == 1 ? 256 : 64 * W) void k_attention_mfma(
 #pragma unroll
                         for (int e = 0; e < E; ++e) sacc[wv][(c * 4 + r) * E + e][lane] = acc[c][e][r];
             }
+            load_k(b + W, k0);
             lds_barrier();
+            if (reg0 < uint32_t(REGS)) {
 #pragma unroll
-            for (int i = 0; i < W; ++i)
-                if ((b0 + i) * 64u < keys) {
-                    l = fmaf(l, alpha[i], ssum[i][col]);
-                    if (reg0 < uint32_t(REGS)) {
+                for (int i = 0; i < W; ++i) {
+                    const bool active = (b0 + i) * 64u < keys;
+                    const float sum = ssum[i][col];
+                    l = active ? fmaf(l, alpha[i], sum) : l;
 #pragma unroll
-                        for (int j = 0; j < R; ++j) o[j] = fmaf(o[j], alpha[i], sacc[i][reg0 + j][lane]);
+                    for (int j = 0; j < R; ++j) {
+                        const float v = sacc[i][reg0 + j][lane];
+                        o[j] = active ? fmaf(o[j], alpha[i], v) : o[j];
                     }
                 }
+            }
             lds_barrier();
         }
         if (raw < total && reg0 < uint32_t(REGS)) {
