@@ -10,6 +10,7 @@
 #include <fstream>
 #include <iterator>
 
+#include "kernels_f32.hpp"
 #include "sha256.hpp"
 
 namespace lrm {
@@ -124,6 +125,7 @@ Device::~Device() {
     lists_.clear();
     for (void* p : pages_)
         if (p) (void)hipFree(p);
+    if (f32_workspace_) (void)hipFree(f32_workspace_);
     for (auto& e : dispatch_events_) {
         (void)hipEventDestroy(e.first);
         (void)hipEventDestroy(e.second);
@@ -146,6 +148,7 @@ void Device::create_heap(const HeapLayout& layout) {
         HIPC(hipMalloc(&pages_[size_t(p.slot)], p.bytes));
         HIPC(hipMemsetAsync(pages_[size_t(p.slot)], 0, p.bytes, stream_));
     }
+    HIPC(hipMalloc(&f32_workspace_, f32k::kWorkspaceBytes));
     HIPC(hipStreamSynchronize(stream_));
     heap_created_ = true;
 }
@@ -285,6 +288,8 @@ void Device::run_probe() {
 
 // ---------------------------------------------------------------- command lists
 
+static constexpr int kAttentionGqaCausal = 13;
+
 CommandList::~CommandList() {
     if (exec_) (void)hipGraphExecDestroy(exec_);
     if (graph_) (void)hipGraphDestroy(graph_);
@@ -310,6 +315,7 @@ void CommandList::dispatch(int kernel, const uint32_t* words) {
         else
             c.ptr[size_t(u.field)] = dev_->resolve(u.token);
     }
+    if (kernel == kAttentionGqaCausal) c.ptr.back() = dev_->f32_workspace_;
     cmds_.push_back(std::move(c));
     ++dispatches_;
 }
@@ -357,6 +363,7 @@ void CommandList::dispatch_library_all(const LibraryDispatch* d, size_t n, const
 void CommandList::dispatch_overlapped(int kernel, const uint32_t* words) {
     dispatch(kernel, words);
     cmds_.back().kind = Cmd::LaunchSide;
+    cmds_.back().ptr.back() = nullptr;  // the workspace is the main stream's
     side_open_ = true;
 }
 

@@ -37,7 +37,8 @@ struct RangeError : std::runtime_error {
 
 void hip_check(hipError_t e, const char* what);
 
-// The launch function of one catalog kernel: pointers per field (nullptr for non-token fields), the prepared words.
+// The launch function of one catalog kernel: pointers per field (nullptr for non-token fields), then the device's float32
+// workspace for the kernel that takes one (nullptr for others, and for overlapped dispatches); the prepared words.
 using LaunchFn = void (*)(const PreparedDispatch& pd, void* const* ptr, hipStream_t stream);
 // One table per kernel source file; entry i is catalog id i or nullptr.
 const LaunchFn* catalog_launchers();  // ids 0..13
@@ -209,6 +210,7 @@ class Device {
     hipEvent_t fork_ev_ = nullptr, join_ev_ = nullptr;
     hipEvent_t epoch_ = nullptr;
     void* static_scratch_ = nullptr;
+    void* f32_workspace_ = nullptr;  // f32k::kWorkspaceBytes, with the heap; main-stream dispatches of id 13 use it in turn
     void* f16_range_[2] = {nullptr, nullptr};
     bool heap_created_ = false;
     HeapLayout layout_;

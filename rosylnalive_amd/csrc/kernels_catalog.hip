@@ -304,7 +304,7 @@ static void l_attention(const PreparedDispatch& pd, void* const* p, hipStream_t 
     uint32_t hd = pd.words[10];
     if (hd > uint32_t(ATT_MAX_HD)) contract_fail("attention_gqa_causal: this device supports head_dim up to %d", ATT_MAX_HD);
     if (f32k::attention((const float*)p[0], (const float*)p[1], (const float*)p[2], (float*)p[3], pd.words[5], pd.words[6],
-                        pd.words[7], pd.words[8], pd.words[9], hd, f32_of(pd.words[11]), s))
+                        pd.words[7], pd.words[8], pd.words[9], hd, f32_of(pd.words[11]), p[11], s))
         return;
     hipLaunchKernelGGL(k_attention_f32, dim3(pd.words[5], pd.words[8]), dim3(64), 0, s, (const float*)p[0],
                        (const float*)p[1], (const float*)p[2], (float*)p[3], pd.words[5], pd.words[6], pd.words[7],

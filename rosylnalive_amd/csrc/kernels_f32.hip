@@ -276,15 +276,14 @@ __device__ __forceinline__ void transpose4(float (&v)[4]) {
     v[3] = __uint_as_float(hi[1]);
 }
 
-__device__ __forceinline__ bool finite(float v) { return (__float_as_uint(v) & 0x7F800000u) != 0x7F800000u; }
-
 template <int HD, int W>
 __global__ __launch_bounds__(W == 1 ? 256 : 64 * W) void k_attention_mfma(
     const float* __restrict__ q, const float* __restrict__ kc, const float* __restrict__ vc, float* __restrict__ y,
     uint32_t rows, uint32_t q_row0, uint32_t past, uint32_t qh, uint32_t kvh, float scale) {
     constexpr int E = HD % 64 == 0 ? 4 : 1, NC = HD / (16 * E), U = HD / 16;
     constexpr int REGS = HD / 4;  // O registers per lane: 16 columns x HD over 64 lanes
-    const uint32_t lane = threadIdx.x & 63u, wv = threadIdx.x >> 6, col = lane & 15u, grp = lane >> 4;
+    const uint32_t lane = threadIdx.x & 63u, wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const uint32_t col = lane & 15u, grp = lane >> 4;
     const uint32_t group = qh / kvh, kvhead = blockIdx.y, total = rows * group, tiles = (total + 15u) / 16u;
     const uint32_t tb = W == 1 ? blockIdx.x * 4u + wv : blockIdx.x;
     if (tb >= tiles) return;
@@ -388,14 +387,14 @@ __global__ __launch_bounds__(W == 1 ? 256 : 64 * W) void k_attention_mfma(
         // a block with such keys holds an infinity or a NaN, each column runs alone with those values zeroed.
         bool odd = false;
         if (b * 64u + 64u > first_keys) {
-            uint32_t bad = 0;
+            float bad = 0.f;  // NaN once a value is not finite
 #pragma unroll
             for (int st = 0; st < 16; ++st)
 #pragma unroll
                 for (int c = 0; c < NC; ++c)
 #pragma unroll
-                    for (int e = 0; e < E; ++e) bad |= uint32_t(!finite(vr[st][c][e]));
-            odd = __ballot(bad != 0u) != 0;
+                    for (int e = 0; e < E; ++e) bad = fmaf(vr[st][c][e], 0.f, bad);
+            odd = __ballot(bad != bad) != 0;
         }
 #pragma unroll
         for (int c = 0; c < NC; ++c)
@@ -553,10 +552,171 @@ __global__ __launch_bounds__(W == 1 ? 256 : 64 * W) void k_attention_mfma(
     }
 }
 
+// One query row (a decode step), G = q_heads / kv_heads of 1, 2 or 4. A workgroup per KV head would use kv_heads CUs, and one
+// CU draws its K and V at about 50 GB/s (8 heads, 700 keys: 36.6 us, 1500: 64.8); so the key blocks spread over the chip,
+// in three launches over a workspace: the scores and the blocks' maxima; the blocks' sums and values against the running
+// maximum (a prefix of those); the ordered combine. The same arithmetic as above, in the same order.
+struct RowWorkspace {
+    float *s, *bmax, *m, *sum, *acc;  // [qh][64 nb], [qh][nb] three times, [qh][nb][HD]
+    __host__ __device__ RowWorkspace(float* base, uint32_t qh, uint32_t nb)
+        : s(base), bmax(s + size_t(qh) * nb * 64), m(bmax + size_t(qh) * nb), sum(m + size_t(qh) * nb),
+          acc(sum + size_t(qh) * nb) {}
+    static uint64_t bytes(uint64_t qh, uint64_t nb, uint64_t hd) { return qh * nb * (67 + hd) * 4; }
+};
+
+// block (key block b, KV head): wave w scores keys 64 b + 16 w .. + 15 for the G heads (a 16-column tile, one chain)
+template <int HD, int G>
+__global__ __launch_bounds__(256) void k_row_scores(const float* __restrict__ q, const float* __restrict__ kc,
+                                                    RowWorkspace ws, uint32_t q_row0, uint32_t past, uint32_t qh,
+                                                    uint32_t kvh, float scale) {
+    constexpr int U = HD / 16;
+    __shared__ float sm[4][16];
+    const uint32_t lane = threadIdx.x & 63u, wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const uint32_t col = lane & 15u, grp = lane >> 4, b = blockIdx.x, nb = gridDim.x, kvhead = blockIdx.y;
+    const uint32_t keys = past + 1u, j0 = b * 64u + 16u * wv, j = j0 + col, head = kvhead * G + col % G;
+    const float* kp = kc + (size_t(j < keys ? j : keys - 1u) * kvh + kvhead) * HD + 4u * grp;
+    const float* qp = q + (size_t(q_row0) * qh + head) * HD + 4u * grp;
+    f32x4 kr[U], qr[U];
+#pragma unroll
+    for (int u = 0; u < U; ++u) kr[u] = *reinterpret_cast<const f32x4*>(kp + 16 * u);
+#pragma unroll
+    for (int u = 0; u < U; ++u) qr[u] = *reinterpret_cast<const f32x4*>(qp + 16 * u);
+    __builtin_amdgcn_sched_barrier(0);
+    float kf[U][4], qf[U][4];
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+            kf[u][i] = kr[u][i];
+            qf[u][i] = qr[u][i];
+        }
+        transpose4(kf[u]);
+        transpose4(qf[u]);
+    }
+    __builtin_amdgcn_sched_barrier(0);
+    f32x4 s = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int u = 0; u < U; ++u)
+#pragma unroll
+        for (int i = 0; i < 4; ++i) s = __builtin_amdgcn_mfma_f32_16x16x4f32(kf[u][i], qf[u][i], s, 0, 0, 0);
+    float mx = -INFINITY;
+#pragma unroll
+    for (int r = 0; r < 4; ++r) {
+        s[r] = j0 + 4u * grp + r < keys ? s[r] * scale : -INFINITY;
+        mx = fmaxf(mx, s[r]);
+    }
+    mx = fast::cross_rows_max(mx);
+    if (lane < 16u) sm[wv][col] = mx;
+    if (col < uint32_t(G)) *reinterpret_cast<f32x4*>(ws.s + size_t(head) * nb * 64 + j0 + 4u * grp) = s;
+    __syncthreads();
+    if (threadIdx.x < uint32_t(G))
+        ws.bmax[size_t(kvhead * G + threadIdx.x) * nb + b] =
+            fmaxf(fmaxf(sm[0][threadIdx.x], sm[1][threadIdx.x]), fmaxf(sm[2][threadIdx.x], sm[3][threadIdx.x]));
+}
+
+// block (key block b, KV head), one thread per head and dimension: the weights against the running maximum, their sum,
+// the block's values
+template <int HD, int G>
+__global__ __launch_bounds__(HD* G < 64 ? 64 : HD * G) void k_row_values(const float* __restrict__ vc, RowWorkspace ws,
+                                                                         uint32_t past, uint32_t kvh) {
+    constexpr int NT = HD * G < 64 ? 64 : HD * G;
+    __shared__ __align__(16) float ps[G][64];
+    const uint32_t t = threadIdx.x, b = blockIdx.x, nb = gridDim.x, kvhead = blockIdx.y;
+    const uint32_t h = t / HD, d = t % HD, keys = past + 1u;
+    const uint32_t count = keys - b * 64u < 64u ? keys - b * 64u : 64u;
+    const float* vp = vc + (size_t(b) * 64u * kvh + kvhead) * HD;
+    float v[64];
+#pragma unroll
+    for (uint32_t j = 0; j < 64; ++j) v[j] = vp[size_t((j < count ? j : count - 1u) * kvh * HD) + d];
+    __builtin_amdgcn_sched_barrier(0);
+    if (t < 64u) {  // one wave: the running maxima, then the weights of key `t`
+#pragma unroll
+        for (int g = 0; g < G; ++g) {
+            const uint32_t head = kvhead * G + g;
+            const float score = ws.s[size_t(head) * nb * 64 + b * 64u + t];
+            float mx = ws.bmax[size_t(head) * nb];
+            for (uint32_t i = t; i <= b; i += 64u) mx = fmaxf(mx, ws.bmax[size_t(head) * nb + i]);
+            mx = fast::wave_max(mx);
+            ps[g][t] = expf(score - mx);
+            if (t == 0) ws.m[size_t(head) * nb + b] = mx;
+        }
+    }
+    lds_barrier();
+    if (h >= uint32_t(G)) return;
+    float acc = 0.f, sum = 0.f;
+    if (count == 64u) {
+#pragma unroll
+        for (int j = 0; j < 64; j += 4) {
+            const f32x4 w = *reinterpret_cast<const f32x4*>(&ps[h][j]);
+#pragma unroll
+            for (int e = 0; e < 4; ++e) {
+                sum += w[e];
+                acc = fmaf(w[e], v[j + e], acc);
+            }
+        }
+    } else {
+#pragma unroll
+        for (uint32_t j = 0; j < 64; ++j)
+            if (j < count) {
+                const float w = ps[h][j];
+                sum += w;
+                acc = fmaf(w, v[j], acc);
+            }
+    }
+    const size_t at = size_t(kvhead * G + h) * nb + b;
+    ws.acc[at * HD + d] = acc;
+    if (d == 0) ws.sum[at] = sum;
+}
+
+// block (query head), one thread per dimension: the blocks in order, 64 at a time
+template <int HD>
+__global__ __launch_bounds__(HD < 64 ? 64 : HD) void k_row_combine(RowWorkspace ws, float* __restrict__ y, uint32_t q_row0,
+                                                                   uint32_t qh, uint32_t nb) {
+    __shared__ float al[64], bs[64];
+    const uint32_t t = threadIdx.x, head = blockIdx.x, d = t % HD;
+    const float* acc = ws.acc + size_t(head) * nb * HD + d;
+    const float* m = ws.m + size_t(head) * nb;
+    float l = 0.f, o = 0.f;
+    for (uint32_t b0 = 0; b0 < nb; b0 += 64u) {
+        if (t < 64u) {
+            const uint32_t b = b0 + t < nb ? b0 + t : nb - 1u;
+            const float before = b == 0 ? ws.bmax[size_t(head) * nb] : m[b - 1u];
+            al[t] = expf(before - m[b]);
+            bs[t] = ws.sum[size_t(head) * nb + b];
+        }
+        __syncthreads();
+        const uint32_t n = nb - b0 < 64u ? nb - b0 : 64u;
+#pragma unroll 8
+        for (uint32_t i = 0; i < n; ++i) {
+            l = fmaf(l, al[i], bs[i]);
+            o = fmaf(o, al[i], acc[size_t(b0 + i) * HD]);
+        }
+        __syncthreads();
+    }
+    if (t < uint32_t(HD)) y[(size_t(q_row0) * qh + head) * HD + d] = o / l;
+}
+
 template <int HD>
 static void launch_attention(const float* q, const float* kc, const float* vc, float* y, uint32_t rows, uint32_t q_row0,
-                             uint32_t past, uint32_t qh, uint32_t kvh, float scale, hipStream_t s) {
+                             uint32_t past, uint32_t qh, uint32_t kvh, float scale, void* workspace,
+                             hipStream_t s) {
     const uint64_t tiles = (uint64_t(rows) * (qh / kvh) + 15) / 16;
+    const uint32_t group = qh / kvh, nb = past / 64u + 1u;
+    // (three launches against one: at 64 and 128 dimensions they win from the first key, 63 keys 10 us against 14; below,
+    // where a block is little work, from eight blocks on)
+    if (workspace && rows == 1 && (HD >= 64 || nb >= 8) && (group == 1 || group == 2 || group == 4) && uint64_t(64) * kvh * HD < (1ull << 30) &&
+        RowWorkspace::bytes(qh, nb, HD) <= kWorkspaceBytes) {
+        const RowWorkspace ws(static_cast<float*>(workspace), qh, nb);
+        auto go = [&](auto scores, auto values, uint32_t threads) {
+            hipLaunchKernelGGL(scores, dim3(nb, kvh), dim3(256), 0, s, q, kc, ws, q_row0, past, qh, kvh, scale);
+            hipLaunchKernelGGL(values, dim3(nb, kvh), dim3(threads < 64 ? 64 : threads), 0, s, vc, ws, past, kvh);
+        };
+        if (group == 1) go(k_row_scores<HD, 1>, k_row_values<HD, 1>, HD);
+        if (group == 2) go(k_row_scores<HD, 2>, k_row_values<HD, 2>, 2 * HD);
+        if (group == 4) go(k_row_scores<HD, 4>, k_row_values<HD, 4>, 4 * HD);
+        hipLaunchKernelGGL(k_row_combine<HD>, dim3(qh), dim3(HD < 64 ? 64 : HD), 0, s, ws, y, q_row0, qh, nb);
+        return;
+    }
     // one wave per tile once the tiles alone fill the chip's 1024 SIMDs several times over; else eight waves share one
     if (tiles * kvh >= 4096)
         hipLaunchKernelGGL((k_attention_mfma<HD, 1>), dim3(uint32_t((tiles + 3) / 4), kvh), dim3(256), 0, s, q, kc, vc, y,
@@ -567,13 +727,13 @@ static void launch_attention(const float* q, const float* kc, const float* vc, f
 }
 
 bool attention(const float* q, const float* kc, const float* vc, float* y, uint32_t rows, uint32_t q_row0, uint32_t past,
-               uint32_t qh, uint32_t kvh, uint32_t hd, float scale, hipStream_t s) {
+               uint32_t qh, uint32_t kvh, uint32_t hd, float scale, void* workspace, hipStream_t s) {
     if (!aligned16(q) || !aligned16(kc) || !aligned16(vc) || uint64_t(rows) * (qh / kvh) > 0x7FFFFFFFull) return false;
     switch (hd) {
-        case 16: launch_attention<16>(q, kc, vc, y, rows, q_row0, past, qh, kvh, scale, s); return true;
-        case 32: launch_attention<32>(q, kc, vc, y, rows, q_row0, past, qh, kvh, scale, s); return true;
-        case 64: launch_attention<64>(q, kc, vc, y, rows, q_row0, past, qh, kvh, scale, s); return true;
-        case 128: launch_attention<128>(q, kc, vc, y, rows, q_row0, past, qh, kvh, scale, s); return true;
+        case 16: launch_attention<16>(q, kc, vc, y, rows, q_row0, past, qh, kvh, scale, workspace, s); return true;
+        case 32: launch_attention<32>(q, kc, vc, y, rows, q_row0, past, qh, kvh, scale, workspace, s); return true;
+        case 64: launch_attention<64>(q, kc, vc, y, rows, q_row0, past, qh, kvh, scale, workspace, s); return true;
+        case 128: launch_attention<128>(q, kc, vc, y, rows, q_row0, past, qh, kvh, scale, workspace, s); return true;
         default: return false;
     }
 }

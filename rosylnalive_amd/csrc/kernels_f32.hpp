@@ -11,9 +11,12 @@ namespace f32k {
 // y[m, n] = x[m, k] . w[n, k]^T (bf16 w), every output one ascending fused chain over k.
 void matmul_bf16w(const float* x, const uint16_t* w, float* y, uint32_t m, uint32_t n, uint32_t k, hipStream_t s);
 
-// attention_gqa_causal on the matrix cores; false (nothing launched) when the shape or an alignment is not covered.
+// attention_gqa_causal on the matrix cores; false (nothing launched) when the shape or an alignment is not covered. A
+// decode row spreads over the chip when `workspace` (kWorkspaceBytes, written by each call, its contents not kept; null:
+// none) holds its blocks: of the 0.6B's 16 heads, up to 21,500 keys.
+constexpr uint64_t kWorkspaceBytes = uint64_t(4) << 20;
 bool attention(const float* q, const float* kc, const float* vc, float* y, uint32_t rows, uint32_t q_row0, uint32_t past,
-               uint32_t qh, uint32_t kvh, uint32_t hd, float scale, hipStream_t s);
+               uint32_t qh, uint32_t kvh, uint32_t hd, float scale, void* workspace, hipStream_t s);
 
 }  // namespace f32k
 }  // namespace lrm
