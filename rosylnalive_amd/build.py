@@ -19,7 +19,8 @@ BUILD = os.path.join(HERE, "_build")
 LIB = os.path.join(HERE, "liblrm_hip.so")
 ROCM = os.environ.get("ROCM_PATH", "/opt/rocm")
 
-HIP_SOURCES = ["kernels_catalog.hip", "kernels_f32.hip", "kernels_fast.hip", "kernels_persist.hip", "scratch_static.hip"]
+HIP_SOURCES = ["kernels_catalog.hip", "kernels_f32.hip", "kernels_fast.hip", "kernels_persist.hip", "scratch_static.hip",
+               "host_io.hip"]
 HOST_SOURCES = ["contract.cpp", "device.cpp", "qwen_exec.cpp", "safetensors.cpp", "tokenizer.cpp", "capi.cpp"]
 
 HIPCC_FLAGS = [

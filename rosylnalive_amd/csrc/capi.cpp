@@ -577,6 +577,7 @@ int lrm_qwen_token(lrm_qwen* q, const char* name, uint32_t* token) {
         need_ptr(q, "model");
         need_ptr(name, "name");
         uint32_t t = q->q.token(name);
+        q->q.expose(name);
         if (token) *token = t;
     });
 }

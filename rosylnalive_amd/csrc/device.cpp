@@ -84,23 +84,7 @@ Device::Device(int index, uint32_t flags) : index_(index), flags_(flags) {
     static_scratch_ = static_scratch_address(index);
     f16_range_[0] = f16_range_word_fast();
     f16_range_[1] = f16_range_word_persist();
-}
-
-uint32_t Device::take_f16_range() {
-    HIPC(hipSetDevice(index_));
-    uint32_t bits = 0;
-    for (void* w : f16_range_) {
-        uint32_t v = 0;
-        HIPC(hipMemcpyAsync(&v, w, 4, hipMemcpyDeviceToHost, stream_));
-        HIPC(hipStreamSynchronize(stream_));
-        if (v) {
-            const uint32_t zero = 0;
-            HIPC(hipMemcpyAsync(w, &zero, 4, hipMemcpyHostToDevice, stream_));
-            HIPC(hipStreamSynchronize(stream_));
-        }
-        bits |= v;
-    }
-    return bits;
+    HIPC(hipHostMalloc(reinterpret_cast<void**>(&host_words_), (kHostIds + kHostIdWords) * 4, hipHostMallocDefault));
 }
 
 std::string f16_range_sites(uint32_t bits) {
@@ -126,6 +110,7 @@ Device::~Device() {
     for (void* p : pages_)
         if (p) (void)hipFree(p);
     if (f32_workspace_) (void)hipFree(f32_workspace_);
+    if (host_words_) (void)hipHostFree(host_words_);
     for (auto& e : dispatch_events_) {
         (void)hipEventDestroy(e.first);
         (void)hipEventDestroy(e.second);
@@ -215,10 +200,11 @@ void* Device::resolve(uint32_t token) const {
 
 // ---------------------------------------------------------------- kernels
 
-static std::array<uint8_t, 32> hash_of_this_library() {
+// (of the file this library was loaded from: once per process)
+static std::array<uint8_t, 32> read_hash_of_this_library() {
     Dl_info dl{};
     std::array<uint8_t, 32> zero{};
-    if (!dladdr(reinterpret_cast<void*>(&hash_of_this_library), &dl) || !dl.dli_fname) return zero;
+    if (!dladdr(reinterpret_cast<void*>(&read_hash_of_this_library), &dl) || !dl.dli_fname) return zero;
     std::ifstream f(dl.dli_fname, std::ios::binary);
     if (!f) return zero;
     std::vector<char> bytes((std::istreambuf_iterator<char>(f)), std::istreambuf_iterator<char>());
@@ -229,7 +215,7 @@ std::array<uint8_t, 32> Device::load_kernels(KernelSet set) {
     if (loaded_) contract_fail("LoadKernels runs exactly once per backend");
     if (set != KernelSet::Reference && set != KernelSet::Fast) contract_fail("unknown kernel set %d", int(set));
     HIPC(hipSetDevice(index_));
-    const std::array<uint8_t, 32> lib = hash_of_this_library();
+    static const std::array<uint8_t, 32> lib = read_hash_of_this_library();
     std::string msg = set == KernelSet::Reference ? "lrm-hip kernel set: reference\n" : "lrm-hip kernel set: fast\n";
     msg.append(reinterpret_cast<const char*>(lib.data()), lib.size());
     shader_hash_ = Sha256::of(msg.data(), msg.size());

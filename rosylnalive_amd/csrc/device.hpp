@@ -189,9 +189,17 @@ class Device {
     int index() const { return index_; }
     // This device's copy of the library's static scratch array (its address from hipGetSymbolAddress at creation)
     void* static_scratch() const { return static_scratch_; }
-    // The fp16 range sites (bits as f16_range_word_fast) that kernels on this GPU flagged since the last call, then
-    // cleared. The words are per GPU, shared by every backend on it; call after the work in question has completed.
-    uint32_t take_f16_range();
+    // Words into device memory in stream order, carried in kernel arguments: nothing is waited for, `src` may go at once.
+    static constexpr size_t kPutWords = 256;
+    void put_words(void* dst, const uint32_t* src, size_t n);
+    // After everything submitted so far: with `range` the fp16 range sites (bits as f16_range_word_fast) that kernels on this GPU
+    // flagged since the last collect, then cleared (the words are per GPU, shared by every backend on it), the argmax
+    // word, the two abort words and the ids (each null: zeros) into the host words, readable once a wait for a later event
+    // or submission has returned, until the next collect.
+    static constexpr uint32_t kHostRange = 0, kHostArgmax = 2, kHostAbort = 3, kHostIds = 8, kHostIdWords = 4096;
+    void collect(bool range, const void* argmax, const void* abort_words, const void* ids, uint32_t nids);
+    const volatile uint32_t* host_words() const { return host_words_; }
+    uint32_t collected_f16_range() const { return host_words()[kHostRange] | host_words()[kHostRange + 1]; }
     void* slot_ptr(int slot) const;
     void* resolve(uint32_t token) const;  // device pointer of a token's first byte
 
@@ -212,6 +220,7 @@ class Device {
     void* static_scratch_ = nullptr;
     void* f32_workspace_ = nullptr;  // f32k::kWorkspaceBytes, with the heap; main-stream dispatches of id 13 use it in turn
     void* f16_range_[2] = {nullptr, nullptr};
+    uint32_t* host_words_ = nullptr;  // pinned, device-visible: kHostIds + kHostIdWords words
     bool heap_created_ = false;
     HeapLayout layout_;
     std::vector<void*> pages_;  // slot i at pages_[i], slot 0 = the table buffer

@@ -205,10 +205,29 @@ QwenExec::QwenExec(Device& dev, const QwenConfig& cfg, const uint32_t* inv_freq_
                  "LRM_HIP_KERNELS_FAST); this one has the reference set");
     plan();
     upload_rope(inv_freq_bits);
+    for (hipEvent_t& e : ev_) hip_check(hipEventCreate(&e), "event");
 }
 
 QwenExec::~QwenExec() {
     if (decode_list_) dev_.release(decode_list_);
+    for (hipEvent_t e : ev_)
+        if (e) (void)hipEventDestroy(e);
+}
+
+void* QwenExec::ptr(const std::string& name) const { return dev_.resolve(token(name)); }
+
+void QwenExec::flush(CommandList*& l) {
+    if (!started_) hip_check(hipEventRecord(ev_[0], dev_.stream()), "event");
+    started_ = true;
+    pieces_.push_back(dev_.submit(l));
+    dev_.release(l);
+    l = dev_.begin();
+}
+
+void QwenExec::settle() {
+    std::vector<uint64_t> p;
+    p.swap(pieces_);
+    for (uint64_t f : p) dev_.wait(f);
 }
 
 void QwenExec::plan() {
@@ -556,9 +575,9 @@ uint32_t QwenExec::forward(int seq, int pos0, const int32_t* ids, int t_, float*
     // yet), up to kMaxSwigluShift; the shift then stays for later calls until a weight changes. Every rerun rewrites the
     // same cache rows and logits.
     for (;;) {
-        am = forward_chunks(seq, pos0, ids, t_, logits, logits_rows);
+        uint32_t bits = 0;
+        am = forward_chunks(seq, pos0, ids, t_, logits, logits_rows, bits);
         if (c.mode != 1) break;
-        const uint32_t bits = dev_.take_f16_range();
         if ((bits & kF16SiteSwiglu) && swiglu_shift_ < kMaxSwigluShift) {
             set_swiglu_shift(swiglu_shift_ + kSwigluShiftStep);
             continue;
@@ -570,12 +589,15 @@ uint32_t QwenExec::forward(int seq, int pos0, const int32_t* ids, int t_, float*
     return am;
 }
 
-uint32_t QwenExec::forward_chunks(int seq, int pos0, const int32_t* ids, int t_, float* logits, int logits_rows) {
+uint32_t QwenExec::forward_chunks(int seq, int pos0, const int32_t* ids, int t_, float* logits, int logits_rows,
+                                  uint32_t& bits) {
     const QwenConfig& c = cfg_;
     uint32_t am = 0xFFFFFFFFu;
     // chunked prefill: max_tokens rows at a time, the cache carrying the earlier chunks
     for (int c0 = 0; c0 < t_; c0 += c.max_tokens) {
         const int n = std::min(c.max_tokens, t_ - c0);
+        started_ = false;
+        f16_bits_ = 0;
         // the requested rows [t - logits_rows, t) that fall in this chunk: a suffix of it, `want` rows long, landing
         // at row `out0` of the caller's buffer
         const int first = std::max(c0, t_ - logits_rows);
@@ -583,13 +605,14 @@ uint32_t QwenExec::forward_chunks(int seq, int pos0, const int32_t* ids, int t_,
         const int out0 = first - (t_ - logits_rows);
         std::vector<uint32_t> u(static_cast<size_t>(n));
         for (int i = 0; i < n; ++i) u[size_t(i)] = uint32_t(ids[c0 + i]);
-        upload_tensor("ids", u.data(), uint64_t(n) * 4);
+        dev_.put_words(ptr("ids"), u.data(), u.size());
         // only the chunks holding some of the requested rows write into the caller's buffer
         float* lg = (logits && want > 0) ? logits + size_t(out0) * c.vocab : nullptr;
         if (c.mode == 1)
             am = forward_fast(seq, pos0 + c0, n, lg, std::max(want, 1));
         else
             am = forward_fp32(pos0 + c0, n, lg, std::max(want, 1));
+        bits |= f16_bits_;
     }
     return am;
 }
@@ -620,11 +643,10 @@ uint32_t QwenExec::forward_fp32(int pos0, int T, float* logits, int lr) {
                    V = c.vocab, HD = c.head_dim, U = uint32_t(T);
     const uint32_t eps = fbits(c.eps);
     const uint32_t scale = fbits(float(std::pow(double(HD), -0.5)));
-    CommandList* l = dev_.begin();
-    hipEvent_t e0, e1;
-    hip_check(hipEventCreate(&e0), "event");
-    hip_check(hipEventCreate(&e1), "event");
     auto tk = [&](const std::string& n) { return token(n); };
+    const uint32_t LR = uint32_t(c.taps ? T : lr);
+    if (LR > dev_.table().row(tk("logits")).count() / V) arg_fail("%u logits rows exceed the logits tensor", LR);
+    CommandList* l = dev_.begin();
     dispatch(l, "embed_gather_bf16", {tk("ids"), tk("model.embed_tokens.weight"), tk("x"), U, H, V});
     tap_copy(l, "embed.out", tk("x"), T, int(H));
     for (int i = 0; i < c.layers; ++i) {
@@ -684,32 +706,28 @@ uint32_t QwenExec::forward_fp32(int pos0, int T, float* logits, int lr) {
         dispatch(l, "add", {tk("r"), tk("dd"), tk("x"), U * H});
         tap_copy(l, p + "out", tk("x"), T, int(H));
         l->barrier();
+        flush(l);
     }
     dispatch(l, "rmsnorm_rows", {tk("x"), tk("model.norm.weight"), tk("f"), U, H, eps});
     tap_copy(l, "final_norm.out", tk("f"), T, int(H));
     l->barrier();
-    const uint32_t LR = uint32_t(c.taps ? T : lr);
-    if (LR > dev_.table().row(tk("logits")).count() / V) arg_fail("%u logits rows exceed the logits tensor", LR);
     dispatch(l, "copy_rows", {tk("f"), tk("f_last"), LR, H, U - LR, 0, H, H});
     l->barrier();
     dispatch(l, "matmul_bf16w", {tk("f_last"), tk("model.embed_tokens.weight"), tk("logits"), LR, V, H});
     if (c.taps) tap_copy(l, "logits", tk("logits"), T, int(V));
     l->barrier();
     dispatch(l, "argmax_rows", {tk("logits"), tk("argmax"), LR, V});
-    hip_check(hipEventRecord(e0, dev_.stream()), "event");
-    uint64_t f = dev_.submit(l);
-    hip_check(hipEventRecord(e1, dev_.stream()), "event");
-    dev_.wait(f);
+    pieces_.push_back(dev_.submit(l));
     dev_.release(l);
-    hip_check(hipEventSynchronize(e1), "event");
+    dev_.collect(false, static_cast<const uint32_t*>(ptr("argmax")) + (LR - 1), nullptr, nullptr, 0);
+    hip_check(hipEventRecord(ev_[1], dev_.stream()), "event");
+    hip_check(hipEventSynchronize(ev_[1]), "event");
+    settle();
     float ms = 0;
-    hip_check(hipEventElapsedTime(&ms, e0, e1), "event");
+    hip_check(hipEventElapsedTime(&ms, ev_[0], ev_[1]), "event");
     last_ms_ = ms;
-    (void)hipEventDestroy(e0);
-    (void)hipEventDestroy(e1);
+    const uint32_t am = dev_.host_words()[Device::kHostArgmax];
     if (logits) download_tensor("logits", logits, uint64_t(lr) * V * 4, uint64_t(LR - uint32_t(lr)) * V * 4);
-    uint32_t am = 0;
-    download_tensor("argmax", &am, 4, uint64_t(LR - 1) * 4);
     return am;
 }
 
@@ -776,6 +794,8 @@ uint32_t QwenExec::forward_fast(int seq, int pos0, int T, float* logits, int lr)
         // on its rows)
         residual_norm("a", p + "down_proj.f16", I,
                       i + 1 < c.layers ? tk(lname(i + 1, kLayerWeights[0])) : tk("model.norm.weight"), ash);
+        // the first layer at once, then every fourth: a submission costs the host about 4 us, recording a layer as much
+        if (i % 4 == 0) flush(l);
     }
     // logits of the last lr rows, LC rows per lm_head dispatch: the final norm over rows r0 .. r0 + n - 1, the lm_head
     // GEMM, and after the last rows the argmax of the last one (the forward returns the last row's id)
@@ -787,45 +807,32 @@ uint32_t QwenExec::forward_fast(int seq, int pos0, int T, float* logits, int lr)
             dispatch(L, "argmax_rows_final", {tk("argmax.partials"), tk("argmax"), 1});
         }
     };
-    // rows that fit one dispatch ride in the layers' list: one submission, so the GPU does not wait for the host
-    // between the last layer and the lm_head (2048-token prefill, last row: 4.11 -> 4.09 ms; 512-token forward with
-    // all its logits: 2.22 -> 2.19 ms)
-    const bool one = uint32_t(lr) <= LC;
-    if (one) lm_head(l, T - lr, uint32_t(lr));
-    hipEvent_t e0, e1;
-    hip_check(hipEventCreate(&e0), "event");
-    hip_check(hipEventCreate(&e1), "event");
-    hip_check(hipEventRecord(e0, dev_.stream()), "event");
-    uint64_t f = dev_.submit(l);
-    if (one) hip_check(hipEventRecord(e1, dev_.stream()), "event");
-    dev_.wait(f);
-    dev_.release(l);
-    uint32_t am = 0;
-    if (one) {
-        hip_check(hipEventSynchronize(e1), "event");
-        download_tensor("argmax", &am, 4, 0);
-        if (logits) download_tensor("logits", logits, uint64_t(lr) * V * 4);
-    }
-    for (int r0 = T - lr; !one && r0 < T; r0 += int(LC)) {
+    // rows that fit one dispatch ride with the layers (no wait before the lm_head); more go a dispatch at a time, the
+    // logits of each downloaded before the next overwrites them
+    uint32_t am = 0, bits = 0;
+    const int first = T - lr;
+    for (int r0 = first; r0 < T; r0 += int(LC)) {
         const uint32_t n = uint32_t(std::min(int(LC), T - r0));
-        CommandList* l2 = dev_.begin();
-        lm_head(l2, r0, n);
-        uint64_t f2 = dev_.submit(l2);
-        dev_.wait(f2);
-        dev_.release(l2);
+        lm_head(l, r0, n);
         const bool last = r0 + int(n) == T;
         if (last) {
-            hip_check(hipEventRecord(e1, dev_.stream()), "event");
-            hip_check(hipEventSynchronize(e1), "event");
-            download_tensor("argmax", &am, 4, 0);
+            pieces_.push_back(dev_.submit(l));
+            dev_.release(l);
+        } else {
+            flush(l);
         }
-        if (logits) download_tensor("logits", logits + size_t(r0 - (T - lr)) * V, uint64_t(n) * V * 4);
+        dev_.collect(true, last ? ptr("argmax") : nullptr, nullptr, nullptr, 0);
+        hip_check(hipEventRecord(ev_[1], dev_.stream()), "event");
+        hip_check(hipEventSynchronize(ev_[1]), "event");
+        settle();
+        bits |= dev_.collected_f16_range();
+        if (last) am = dev_.host_words()[Device::kHostArgmax];
+        if (logits) download_tensor("logits", logits + size_t(r0 - first) * V, uint64_t(n) * V * 4);
     }
+    f16_bits_ |= bits;
     float ms = 0;
-    hip_check(hipEventElapsedTime(&ms, e0, e1), "event");
+    hip_check(hipEventElapsedTime(&ms, ev_[0], ev_[1]), "event");
     last_ms_ = ms;
-    (void)hipEventDestroy(e0);
-    (void)hipEventDestroy(e1);
     return am;
 }
 
@@ -938,76 +945,105 @@ void QwenExec::record_decode_batch(CommandList* l) {
 void QwenExec::set_decode_state(const int32_t* ids, const int32_t* pos) {
     if (cfg_.mode != 1) arg_fail("on-device decode needs the fast mode");
     const int B = cfg_.batch;
-    std::vector<uint32_t> st(size_t(2 * B + 2), 0u);
-    for (int b = 0; b < B; ++b) {
+    for (int b = 0; b < B; ++b)
         if (pos[b] < 0 || pos[b] >= cfg_.max_pos) arg_fail("decode position %d outside max_pos %d", pos[b], cfg_.max_pos);
-        st[size_t(b)] = uint32_t(pos[b]);
-        st[size_t(B + b)] = uint32_t(ids[b]);
-    }
-    upload_tensor("dec.state", st.data(), st.size() * 4);
+    put_state(ids, pos, 0);
     if (persist_) {
         // After an aborted step the exchange entries are in an unknown mix of steps: start over from zeros (epoch 0,
         // every entry untagged); otherwise the entries of the last step carry its tag, which the next launch's differs
         // from. LRM_HIP_PERSIST_WAIT_US bounds each wait of the step's workgroups (default 0.2 s): a tiny bound makes
         // steps abort, which is how the failure path is tested.
-        uint32_t hdr[4];
-        download_tensor("dec.exchange", hdr, sizeof hdr);
-        if (hdr[1]) {
-            std::vector<uint8_t> zero(dev_.table().row(token("dec.exchange")).extent_bytes(), 0);
-            upload_tensor("dec.exchange", zero.data(), zero.size());
-            hdr[0] = hdr[1] = hdr[2] = 0u;
+        if (persist_aborted_ || dec_exposed_) {
+            uint32_t hdr[4];
+            download_tensor("dec.exchange", hdr, sizeof hdr);
+            if (hdr[1]) {
+                std::vector<uint8_t> zero(dev_.table().row(token("dec.exchange")).extent_bytes(), 0);
+                upload_tensor("dec.exchange", zero.data(), zero.size());
+                hdr[3] = 0u;
+            }
+            persist_wait_ = hdr[3];
+            persist_aborted_ = false;
         }
         const char* w = std::getenv("LRM_HIP_PERSIST_WAIT_US");
         const long us = w ? std::strtol(w, nullptr, 10) : 0;
-        hdr[3] = us > 0 ? uint32_t(std::min<long>(us, 40000000L) * 100) : 0u;
-        upload_tensor("dec.exchange", hdr, sizeof hdr);
+        const uint32_t bound = us > 0 ? uint32_t(std::min<long>(us, 40000000L) * 100) : 0u;
+        if (bound != persist_wait_) dev_.put_words(static_cast<uint32_t*>(ptr("dec.exchange")) + 3, &bound, 1);
+        persist_wait_ = bound;
     }
+}
+
+// pos[b], id[b], the step index, and the spare word, on the device and as the host's copy
+void QwenExec::put_state(const int32_t* ids, const int32_t* pos, uint32_t step) {
+    const int B = cfg_.batch;
+    std::vector<uint32_t> st(size_t(2 * B + 2), 0u);
+    for (int b = 0; b < B; ++b) {
+        st[size_t(b)] = uint32_t(pos[b]);
+        st[size_t(B + b)] = uint32_t(ids[b]);
+    }
+    st[size_t(2 * B)] = step;
+    dev_.put_words(ptr("dec.state"), st.data(), st.size());
+    dec_state_ = std::move(st);
+    dec_ids_ = 0;
 }
 
 void QwenExec::run_decode_steps(int steps) {
     if (cfg_.mode != 1) arg_fail("on-device decode needs the fast mode");
     if (steps < 1) return;
     const int B = cfg_.batch;
-    std::vector<uint32_t> st(size_t(2 * B + 2));
-    download_tensor("dec.state", st.data(), st.size() * 4);
+    if (dec_exposed_) dec_state_.clear();
+    std::vector<uint32_t> st;
+    st.swap(dec_state_);  // (not known again until this run has succeeded)
+    dec_ids_ = 0;
+    if (st.empty()) {
+        st.resize(size_t(2 * B + 2));
+        download_tensor("dec.state", st.data(), st.size() * 4);
+    }
     for (int b = 0; b < B; ++b)
         if (int64_t(st[size_t(b)]) + steps > cfg_.max_pos)
             arg_fail("%d decode steps from position %u pass max_pos %d", steps, st[size_t(b)], cfg_.max_pos);
     if (!decode_list_) record_decode_fast();
     sync_f16();  // the batched step's skinny GEMMs read the fp16 copies: weights set since the last forward
-    hipEvent_t e0, e1;
-    hip_check(hipEventCreate(&e0), "event");
-    hip_check(hipEventCreate(&e1), "event");
-    hip_check(hipEventRecord(e0, dev_.stream()), "event");
+    hip_check(hipEventRecord(ev_[0], dev_.stream()), "event");
     uint64_t f = dev_.submit(decode_list_, uint32_t(steps));
-    hip_check(hipEventRecord(e1, dev_.stream()), "event");
+    // the ids of this sequence of runs so far, where they fit
+    const uint64_t total = (uint64_t(st[size_t(2 * B)]) + uint64_t(steps)) * uint64_t(B);
+    const uint32_t nids = dec_exposed_ || total > Device::kHostIdWords ? 0u : uint32_t(total);
+    dev_.collect(true, nullptr, persist_ ? static_cast<const uint32_t*>(ptr("dec.exchange")) + 1 : nullptr, ptr("dec.out_ids"),
+                 nids);
+    hip_check(hipEventRecord(ev_[1], dev_.stream()), "event");
+    hip_check(hipEventSynchronize(ev_[1]), "event");
     dev_.wait(f);
-    hip_check(hipEventSynchronize(e1), "event");
     float ms = 0;
-    hip_check(hipEventElapsedTime(&ms, e0, e1), "event");
+    hip_check(hipEventElapsedTime(&ms, ev_[0], ev_[1]), "event");
     last_ms_ = ms;
-    (void)hipEventDestroy(e0);
-    (void)hipEventDestroy(e1);
     if (persist_) {  // a workgroup that waited past its bound aborted the step (and every later one)
-        uint32_t hdr[3];
-        download_tensor("dec.exchange", hdr, sizeof hdr);
-        if (hdr[1] && hdr[2] == uint32_t(persist::kStageClaim))
+        const uint32_t aborted = dev_.host_words()[Device::kHostAbort], stage = dev_.host_words()[Device::kHostAbort + 1];
+        persist_aborted_ = persist_aborted_ || aborted != 0;
+        if (aborted && stage == uint32_t(persist::kStageClaim))
             throw std::runtime_error("decode_step_persistent: two workgroups of one launch took the same (XCD, role) "
                                      "slot (the dispatcher placed the workgroups otherwise than the step assumes); "
                                      "the step's results are not valid");
-        if (hdr[1])
+        if (aborted)
             throw std::runtime_error("decode_step_persistent: a workgroup waited past its bound at stage " +
-                                     std::to_string(hdr[2]) + "; the decode state did not advance from there");
+                                     std::to_string(stage) + "; the decode state did not advance from there");
     }
     // A decode call cannot rerun (its steps advanced the state): it fails, and a SwiGLU overflow raises the shift
     // for the calls after it.
-    const uint32_t bits = dev_.take_f16_range();
+    const uint32_t bits = dev_.collected_f16_range();
     if (bits & kF16SiteSwiglu) set_swiglu_shift(std::min(kMaxSwigluShift, swiglu_shift_ + kSwigluShiftStep));
     if (bits) throw_f16_range("decode", bits);
+    for (int b = 0; b < B; ++b) st[size_t(b)] += uint32_t(steps);
+    st[size_t(2 * B)] += uint32_t(steps);
+    dec_state_ = std::move(st);
+    dec_ids_ = int(nids);
 }
 
 void QwenExec::read_decode_ids(int32_t* out, int count) {
     if (count < 0 || int64_t(count) > int64_t(cfg_.max_pos) * cfg_.batch) arg_fail("count %d", count);
+    if (count <= dec_ids_ && !dec_exposed_) {
+        for (int i = 0; i < count; ++i) out[i] = int32_t(dev_.host_words()[Device::kHostIds + uint32_t(i)]);
+        return;
+    }
     download_tensor("dec.out_ids", out, uint64_t(count) * 4);
 }
 
@@ -1024,8 +1060,7 @@ void QwenExec::greedy(const int32_t* prompt, int plen, int steps, int32_t* out) 
         int32_t pos = plen;
         int32_t i0 = int32_t(id);
         set_decode_state(&i0, &pos);
-        uint32_t st[4] = {uint32_t(plen), id, 1, 0};
-        upload_tensor("dec.state", st, 16);
+        put_state(&i0, &pos, 1);
         run_decode_steps(steps - 1);
         std::vector<int32_t> ids(static_cast<size_t>(steps));
         read_decode_ids(ids.data(), steps);

@@ -75,6 +75,8 @@ class QwenExec {
     const QwenConfig& config() const { return cfg_; }
     Device& device() { return dev_; }
     uint32_t token(const std::string& name) const;
+    // A caller that asks for the decode state's tensors may write them: the host's copies are not used from there on.
+    void expose(const std::string& name) { dec_exposed_ = dec_exposed_ || name.rfind("dec.", 0) == 0; }
     void run_decode_steps(int steps);  // Fast mode: replays the recorded decode step `steps` times (state on device)
     void set_decode_state(const int32_t* ids, const int32_t* pos);
     void read_decode_ids(int32_t* out, int count);
@@ -98,7 +100,13 @@ class QwenExec {
     void upload_rope(const uint32_t* inv_freq_bits);
     uint32_t forward_fp32(int pos0, int t, float* logits, int logits_rows);
     uint32_t forward_fast(int seq, int pos0, int t, float* logits, int logits_rows);
-    uint32_t forward_chunks(int seq, int pos0, const int32_t* ids, int t, float* logits, int logits_rows);
+    // bits: the fp16 range sites of all chunks
+    uint32_t forward_chunks(int seq, int pos0, const int32_t* ids, int t, float* logits, int logits_rows, uint32_t& bits);
+    // A forward's dispatches go out in pieces, so that the GPU works while the host records the rest: flush submits what
+    // `l` holds and begins the next piece, settle waits for every piece.
+    void flush(CommandList*& l);
+    void settle();
+    void put_state(const int32_t* ids, const int32_t* pos, uint32_t step);
     void set_swiglu_shift(int s);
     void set_weight_bytes(const std::string& name, const uint8_t* data, uint64_t elems);
     // Fast mode: fails the call (RangeError) naming the fp16 range sites in bits.
@@ -130,6 +138,16 @@ class QwenExec {
     int last_t_ = 0;
     double last_ms_ = 0;
     CommandList* decode_list_ = nullptr;
+    bool started_ = false;                         // the running forward's first piece is out
+    uint32_t f16_bits_ = 0;                        // the running forward's fp16 range sites
+    std::vector<uint64_t> pieces_;                 // submissions of the running forward
+    hipEvent_t ev_[2] = {nullptr, nullptr};        // around the device work that last_ms() reports
+    std::vector<uint32_t> dec_state_;              // the device's decode state as the host knows it; empty: not known
+    int dec_ids_ = 0;                              // ids of the last run in the device's host words
+    bool dec_exposed_ = false;
+    bool persist_aborted_ = false;                 // the last persistent run aborted: the exchange area starts over
+    uint32_t persist_wait_ = 0;                    // the wait bound the exchange header holds
+    void* ptr(const std::string& name) const;      // device pointer of a tensor
     bool persist_ = false;    // the decode step is decode_step_persistent (layer-stacked weights and caches)
     int persist_blocks_ = 0;  // its workgroups
     int swiglu_shift_ = 0;
