@@ -447,14 +447,88 @@ static std::vector<KernelSpec> base_catalog() {
     return c;
 }
 
-// The appended entries of this backend (ids 14 and up), defined next to their kernels' host code.
+// The appended entries of this backend: the fast path (ids 14..40), defined next to its kernels' host code, then fusions
+// of the reference's own kernels (ids 41..44), whose results equal the dispatches they stand for bit for bit.
 std::vector<KernelSpec> fast_catalog();
+
+static std::vector<KernelSpec> fused_catalog() {
+    std::vector<KernelSpec> c;
+    // 41 matmul_bf16w_triple: x, w0, w1, w2, y0, y1, y2, m, n0, n1, n2, k: three matmul_bf16w of one x
+    c.push_back({"matmul_bf16w_triple", "matmul", {256, 1, 1}, false,
+                 [](const uint32_t* w) {
+                     return Grid3{cdiv(w[9], 64) + cdiv(w[10], 64) + cdiv(w[11], 64), cdiv(w[8], 64), 1};
+                 },
+                 {TOK_R("x", DT(F32)), TOK_R("w0", DT(BF16)), TOK_R("w1", DT(BF16)), TOK_R("w2", DT(BF16)),
+                  TOK_W("y0", DT(F32), nullptr), TOK_W("y1", DT(F32), nullptr), TOK_W("y2", DT(F32), nullptr), U32F("m"),
+                  U32F("n0"), U32F("n1"), U32F("n2"), U32F("k")},
+                 [](const uint32_t* w, const uint32_t* c) {
+                     need(c, 0, int64_t(w[8]) * w[12], "matmul_bf16w_triple", "x");
+                     for (int i = 0; i < 3; ++i) {
+                         if (w[9 + i] < 1) contract_fail("matmul_bf16w_triple: n must be at least 1");
+                         need(c, 1 + i, int64_t(w[9 + i]) * w[12], "matmul_bf16w_triple", "w");
+                         need(c, 4 + i, int64_t(w[8]) * w[9 + i], "matmul_bf16w_triple", "y");
+                     }
+                 }});
+    // 42 matmul_bf16w_pair: x, w0, w1, y0, y1, m, n0, n1, k
+    c.push_back({"matmul_bf16w_pair", "matmul", {256, 1, 1}, false,
+                 [](const uint32_t* w) { return Grid3{cdiv(w[7], 64) + cdiv(w[8], 64), cdiv(w[6], 64), 1}; },
+                 {TOK_R("x", DT(F32)), TOK_R("w0", DT(BF16)), TOK_R("w1", DT(BF16)), TOK_W("y0", DT(F32), nullptr),
+                  TOK_W("y1", DT(F32), nullptr), U32F("m"), U32F("n0"), U32F("n1"), U32F("k")},
+                 [](const uint32_t* w, const uint32_t* c) {
+                     need(c, 0, int64_t(w[6]) * w[9], "matmul_bf16w_pair", "x");
+                     for (int i = 0; i < 2; ++i) {
+                         if (w[7 + i] < 1) contract_fail("matmul_bf16w_pair: n must be at least 1");
+                         need(c, 1 + i, int64_t(w[7 + i]) * w[9], "matmul_bf16w_pair", "w");
+                         need(c, 3 + i, int64_t(w[6]) * w[7 + i], "matmul_bf16w_pair", "y");
+                     }
+                 }});
+    // 43 qk_norm_rope_append: rmsnorm_rows and rope_apply on q's and k's heads, copy_rows of k and v into the caches' rows
+    // pos0 ..
+    c.push_back({"qk_norm_rope_append", "attention", {256, 1, 1}, false,
+                 [](const uint32_t* w) { return Grid3{w[11], int64_t(w[12]) + 2 * int64_t(w[13]), 1}; },
+                 {TOK_R("q", DT(F32)), TOK_R("k", DT(F32)), TOK_R("v", DT(F32)), TOK_R("q_norm", DT(BF16)),
+                  TOK_R("k_norm", DT(BF16)), TOK_R("cos_table", DT(F32)), TOK_R("sin_table", DT(F32)),
+                  TOK_W("qr", DT(F32), nullptr), TOK_W("k_cache", DT(F32), nullptr), TOK_W("v_cache", DT(F32), nullptr),
+                  U32F("rows"), U32F("q_heads"), U32F("kv_heads"), U32F("head_dim"), U32F("pos0"), F32F("eps")},
+                 [](const uint32_t* w, const uint32_t* c) {
+                     const char* n = "qk_norm_rope_append";
+                     const int64_t rows = w[11], qh = w[12], kvh = w[13], hd = w[14], pos0 = w[15];
+                     if (qh < 1 || kvh < 1) contract_fail("%s: heads must be at least 1", n);
+                     if (hd < 2 || hd % 2 || hd > 8192) contract_fail("%s: head_dim must be even, 2 to 8192", n);
+                     need(c, 0, rows * qh * hd, n, "q");
+                     need(c, 1, rows * kvh * hd, n, "k");
+                     need(c, 2, rows * kvh * hd, n, "v");
+                     need(c, 3, hd, n, "q_norm");
+                     need(c, 4, hd, n, "k_norm");
+                     need(c, 5, (pos0 + rows) * (hd / 2), n, "cos_table");
+                     need(c, 6, (pos0 + rows) * (hd / 2), n, "sin_table");
+                     need(c, 7, rows * qh * hd, n, "qr");
+                     need(c, 8, (pos0 + rows) * kvh * hd, n, "k_cache");
+                     need(c, 9, (pos0 + rows) * kvh * hd, n, "v_cache");
+                 }});
+    // 44 add_rmsnorm_rows: r = a + b (add), y = rmsnorm_rows(r, w)
+    c.push_back({"add_rmsnorm_rows", "basic", {256, 1, 1}, true, [](const uint32_t* w) { return Grid3{w[6], 1, 1}; },
+                 {TOK_R("a", DT(F32)), TOK_R("b", DT(F32)), TOK_R("w", DT(BF16)), TOK_W("r", DT(F32), nullptr),
+                  TOK_W("y", DT(F32), nullptr), U32F("rows"), U32F("cols"), F32F("eps")},
+                 [](const uint32_t* w, const uint32_t* c) {
+                     if (w[7] < 1) contract_fail("add_rmsnorm_rows: cols must be at least 1");
+                     const int64_t n = int64_t(w[6]) * w[7];
+                     need(c, 0, n, "add_rmsnorm_rows", "a");
+                     need(c, 1, n, "add_rmsnorm_rows", "b");
+                     need(c, 2, w[7], "add_rmsnorm_rows", "w");
+                     need(c, 3, n, "add_rmsnorm_rows", "r");
+                     need(c, 4, n, "add_rmsnorm_rows", "y");
+                 }});
+    return c;
+}
 
 const std::vector<KernelSpec>& catalog() {
     static const std::vector<KernelSpec> all = [] {
         auto c = base_catalog();
         auto f = fast_catalog();
         c.insert(c.end(), f.begin(), f.end());
+        auto u = fused_catalog();
+        c.insert(c.end(), u.begin(), u.end());
         return c;
     }();
     return all;

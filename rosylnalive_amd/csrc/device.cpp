@@ -227,12 +227,14 @@ std::array<uint8_t, 32> Device::load_kernels(KernelSet set) {
 
 bool Device::contains(int kernel) const {
     if (kernel < 0 || kernel >= catalog_size()) return false;
+    if (kernel >= kFusedFirstId) return true;  // both sets: the bits of the reference kernels they stand for
     if (set_ == KernelSet::Reference && kernel >= fast_first_id()) return false;
     if (kernel < fast_first_id()) return catalog_launchers()[kernel] != nullptr;
     return fast_launchers()[kernel - fast_first_id()] != nullptr;
 }
 
 static LaunchFn launcher_of(int kernel) {
+    if (kernel >= kFusedFirstId) return fused_launchers()[kernel - kFusedFirstId];
     return kernel < fast_first_id() ? catalog_launchers()[kernel] : fast_launchers()[kernel - fast_first_id()];
 }
 

@@ -42,8 +42,10 @@ void hip_check(hipError_t e, const char* what);
 using LaunchFn = void (*)(const PreparedDispatch& pd, void* const* ptr, hipStream_t stream);
 // One table per kernel source file; entry i is catalog id i or nullptr.
 const LaunchFn* catalog_launchers();  // ids 0..13
-const LaunchFn* fast_launchers();     // ids 14..
+const LaunchFn* fast_launchers();     // ids 14..40
 int fast_first_id();
+const LaunchFn* fused_launchers();    // ids 41.. (kFusedFirstId)
+constexpr int kFusedFirstId = 41;
 
 class Device;
 class CommandList;

@@ -1,6 +1,7 @@
 // The reference catalog's kernels 0..13 (docs/contracts/kernel-abi.md "The catalog at contracts-v1") for gfx950:
 // fp32 activations, bf16 weights, the arithmetic of CpuRef F32 where the catalog asks for it. These are the parity
-// path of the device (the executor's fp32 mode); the bf16 performance kernels are in kernels_fast.hip.
+// path of the device (the executor's fp32 mode), with its contractions in kernels_f32.hip and, at the end of the catalog
+// (ids 41..44), fusions of it with the same bits; the bf16 performance kernels are in kernels_fast.hip.
 //
 // Built with -ffp-contract=off: every product is rounded before the following add unless fmaf is written, as CpuRef
 // does (docs/contracts/cpu-reference.md rules 2 and 4). Division and sqrtf are IEEE (hipcc's default
@@ -135,11 +136,99 @@ __global__ void k_copy_rows(const uint32_t* src, uint32_t* dst, uint32_t rows, u
     dst[(uint64_t(dr0) + r) * ds + c] = src[(uint64_t(sr0) + r) * ss + c];
 }
 
+// ================================================================ fusions (ids 41..44)
+// The float32 forward's runs of small dispatches as one launch each (a launch costs 2-5 us, most of these kernels' time),
+// with the arithmetic of the kernels they replace, operation for operation.
+
+// ---------------------------------------------------------------- 43 qk_norm_rope_append
+// One block per (row, head of q, k or v): rmsnorm_rows on the head, rope_apply, and the row's place: qr for q, the caches
+// for k and v (v as it is).
+__global__ __launch_bounds__(256) void k_qk_norm_rope_append(const float* q, const float* k, const float* v,
+                                                             const uint16_t* qn, const uint16_t* kn, const float* cos_t,
+                                                             const float* sin_t, float* qr, float* kc, float* vc,
+                                                             uint32_t qh, uint32_t kvh, uint32_t hd, uint32_t pos0,
+                                                             float eps) {
+    __shared__ float red[4];
+    extern __shared__ float xn[];  // the normed head
+    const uint32_t r = blockIdx.x, h = blockIdx.y, half = hd / 2u;
+    const size_t pos = size_t(pos0) + r;
+    if (h >= qh + kvh) {
+        const size_t at = h - qh - kvh;
+        for (uint32_t c = threadIdx.x; c < hd; c += 256u) vc[(pos * kvh + at) * hd + c] = v[(size_t(r) * kvh + at) * hd + c];
+        return;
+    }
+    const bool is_q = h < qh;
+    const float* xr = is_q ? q + (size_t(r) * qh + h) * hd : k + (size_t(r) * kvh + (h - qh)) * hd;
+    const uint16_t* w = is_q ? qn : kn;
+    float* yr = is_q ? qr + (size_t(r) * qh + h) * hd : kc + (pos * kvh + (h - qh)) * hd;
+    float ss = 0.f;
+    for (uint32_t c = threadIdx.x; c < hd; c += 256u) ss = fmaf(xr[c], xr[c], ss);
+    ss = block_sum_256(ss, red);
+    const float mean = ss / float(hd);
+    const float rr = 1.0f / sqrtf(mean + eps);
+    for (uint32_t c = threadIdx.x; c < hd; c += 256u) {
+        const float xv = xr[c] * rr;
+        xn[c] = widen(w[c]) * xv;
+    }
+    __syncthreads();
+    for (uint32_t i = threadIdx.x; i < half; i += 256u) {
+        const float c = cos_t[pos * half + i], s = sin_t[pos * half + i];
+        const float a = xn[i], b = xn[i + half];
+        const float ac = a * c, bs = b * s, bc = b * c, as = a * s;
+        yr[i] = ac - bs;
+        yr[i + half] = bc + as;
+    }
+}
+
+// ---------------------------------------------------------------- 44 add_rmsnorm_rows: r = a + b, y = rmsnorm_rows(r)
+__global__ __launch_bounds__(256) void k_add_rmsnorm_rows(const float* a, const float* b, const uint16_t* w, float* r,
+                                                          float* y, uint32_t rows, uint32_t cols, float eps) {
+    __shared__ float red[4];
+    const uint32_t row = linear_group();
+    if (row >= rows) return;
+    const size_t at = size_t(row) * cols;
+    constexpr int KEEP = 8;  // of the row's sums per thread (2048 columns); the rest are read back
+    float x[KEEP];
+    float ss = 0.f;
+#pragma unroll
+    for (int i = 0; i < KEEP; ++i) {
+        const uint32_t c = threadIdx.x + 256u * i;
+        if (c < cols) {
+            x[i] = a[at + c] + b[at + c];
+            r[at + c] = x[i];
+            ss = fmaf(x[i], x[i], ss);
+        }
+    }
+    for (uint32_t c = threadIdx.x + 256u * KEEP; c < cols; c += 256u) {
+        const float v = a[at + c] + b[at + c];
+        r[at + c] = v;
+        ss = fmaf(v, v, ss);
+    }
+    ss = block_sum_256(ss, red);
+    const float mean = ss / float(cols);
+    const float rr = 1.0f / sqrtf(mean + eps);
+#pragma unroll
+    for (int i = 0; i < KEEP; ++i) {
+        const uint32_t c = threadIdx.x + 256u * i;
+        if (c < cols) {
+            const float xv = x[i] * rr;
+            y[at + c] = widen(w[c]) * xv;
+        }
+    }
+    for (uint32_t c = threadIdx.x + 256u * KEEP; c < cols; c += 256u) {
+        const float xv = r[at + c] * rr;
+        y[at + c] = widen(w[c]) * xv;
+    }
+}
+
 // ---------------------------------------------------------------- 11 argmax_rows
 // The lowest index of the row maximum by '>' (+0 and -0 tie); a row holding a NaN gives 0xFFFFFFFF.
-__global__ void k_argmax_rows(const float* x, uint32_t* y, uint32_t rows, uint32_t cols) {
-    __shared__ float sv[256];
-    __shared__ uint32_t si[256];
+// 1024 threads with four loads in flight each: a row's time is its loads' latency (4,096 columns: 7.1 us with 256 threads,
+// one load at a time).
+constexpr uint32_t AM_T = 1024;
+__global__ __launch_bounds__(1024) void k_argmax_rows(const float* x, uint32_t* y, uint32_t rows, uint32_t cols) {
+    __shared__ float sv[AM_T];
+    __shared__ uint32_t si[AM_T];
     __shared__ int snan;
     uint32_t r = linear_group();
     if (r >= rows) return;
@@ -149,19 +238,24 @@ __global__ void k_argmax_rows(const float* x, uint32_t* y, uint32_t rows, uint32
     float best = 0.f;
     uint32_t bi = 0xFFFFFFFFu;
     bool nan = false;
-    for (uint32_t c = threadIdx.x; c < cols; c += 256u) {
-        float v = xr[c];
-        if (v != v) nan = true;
-        else if (bi == 0xFFFFFFFFu || v > best) {
-            best = v;
-            bi = c;
+    for (uint64_t c0 = threadIdx.x; c0 < cols; c0 += 4 * AM_T) {
+        float v[4];
+#pragma unroll
+        for (uint32_t e = 0; e < 4; ++e) v[e] = xr[c0 + e * AM_T < cols ? c0 + e * AM_T : c0];  // (past the row: again)
+#pragma unroll
+        for (uint32_t e = 0; e < 4; ++e) {
+            if (v[e] != v[e]) nan = true;
+            else if (bi == 0xFFFFFFFFu || v[e] > best) {
+                best = v[e];
+                bi = uint32_t(c0 + e * AM_T);
+            }
         }
     }
     if (nan) atomicOr(&snan, 1);
     sv[threadIdx.x] = best;
     si[threadIdx.x] = bi;
     __syncthreads();
-    for (uint32_t s = 128; s > 0; s >>= 1) {
+    for (uint32_t s = AM_T / 2; s > 0; s >>= 1) {
         if (threadIdx.x < s) {
             float ov = sv[threadIdx.x + s];
             uint32_t oi = si[threadIdx.x + s];
@@ -295,10 +389,11 @@ static void l_copy_rows(const PreparedDispatch& pd, void* const* p, hipStream_t 
                        pd.words[4], pd.words[5], pd.words[6], pd.words[7], pd.words[8]);
 }
 static void l_argmax(const PreparedDispatch& pd, void* const* p, hipStream_t s) {
-    hipLaunchKernelGGL(k_argmax_rows, phys(pd), dim3(256), 0, s, (const float*)p[0], (uint32_t*)p[1], pd.words[3], pd.words[4]);
+    hipLaunchKernelGGL(k_argmax_rows, phys(pd), dim3(AM_T), 0, s, (const float*)p[0], (uint32_t*)p[1], pd.words[3], pd.words[4]);
 }
 static void l_matmul(const PreparedDispatch& pd, void* const* p, hipStream_t s) {
-    f32k::matmul_bf16w((const float*)p[0], (const uint16_t*)p[1], (float*)p[2], pd.words[4], pd.words[5], pd.words[6], s);
+    const f32k::MatmulGroup g{{(const uint16_t*)p[1], nullptr, nullptr}, {(float*)p[2], nullptr, nullptr}, {pd.words[5], 0, 0}, 1};
+    f32k::matmul_bf16w((const float*)p[0], g, pd.words[4], pd.words[6], s);
 }
 static void l_attention(const PreparedDispatch& pd, void* const* p, hipStream_t s) {
     uint32_t hd = pd.words[10];
@@ -309,6 +404,44 @@ static void l_attention(const PreparedDispatch& pd, void* const* p, hipStream_t 
     hipLaunchKernelGGL(k_attention_f32, dim3(pd.words[5], pd.words[8]), dim3(64), 0, s, (const float*)p[0],
                        (const float*)p[1], (const float*)p[2], (float*)p[3], pd.words[5], pd.words[6], pd.words[7],
                        pd.words[8], pd.words[9], hd, f32_of(pd.words[11]));
+}
+
+// 41 matmul_bf16w_triple: x, w0, w1, w2, y0, y1, y2, m, n0, n1, n2, k
+static void l_matmul_triple(const PreparedDispatch& pd, void* const* p, hipStream_t s) {
+    const uint32_t* w = pd.words.data();
+    const f32k::MatmulGroup g{{(const uint16_t*)p[1], (const uint16_t*)p[2], (const uint16_t*)p[3]},
+                              {(float*)p[4], (float*)p[5], (float*)p[6]},
+                              {w[9], w[10], w[11]},
+                              3};
+    f32k::matmul_bf16w((const float*)p[0], g, w[8], w[12], s);
+}
+// 42 matmul_bf16w_pair: x, w0, w1, y0, y1, m, n0, n1, k
+static void l_matmul_pair(const PreparedDispatch& pd, void* const* p, hipStream_t s) {
+    const uint32_t* w = pd.words.data();
+    const f32k::MatmulGroup g{{(const uint16_t*)p[1], (const uint16_t*)p[2], nullptr},
+                              {(float*)p[3], (float*)p[4], nullptr},
+                              {w[7], w[8], 0},
+                              2};
+    f32k::matmul_bf16w((const float*)p[0], g, w[6], w[9], s);
+}
+// 43 qk_norm_rope_append: q, k, v, q_norm, k_norm, cos, sin, qr, k_cache, v_cache, rows, q_heads, kv_heads, head_dim, pos0, eps
+static void l_qk_norm_rope_append(const PreparedDispatch& pd, void* const* p, hipStream_t s) {
+    const uint32_t* w = pd.words.data();
+    hipLaunchKernelGGL(k_qk_norm_rope_append, dim3(w[11], w[12] + 2 * w[13]), dim3(256), w[14] * 4, s, (const float*)p[0],
+                       (const float*)p[1], (const float*)p[2], (const uint16_t*)p[3], (const uint16_t*)p[4],
+                       (const float*)p[5], (const float*)p[6], (float*)p[7], (float*)p[8], (float*)p[9], w[12], w[13],
+                       w[14], w[15], f32_of(w[16]));
+}
+// 44 add_rmsnorm_rows: a, b, w, r, y, rows, cols, eps
+static void l_add_rmsnorm(const PreparedDispatch& pd, void* const* p, hipStream_t s) {
+    const uint32_t* w = pd.words.data();
+    hipLaunchKernelGGL(k_add_rmsnorm_rows, phys(pd), dim3(256), 0, s, (const float*)p[0], (const float*)p[1],
+                       (const uint16_t*)p[2], (float*)p[3], (float*)p[4], w[6], w[7], f32_of(w[8]));
+}
+
+const LaunchFn* fused_launchers() {
+    static const LaunchFn t[4] = {l_matmul_triple, l_matmul_pair, l_qk_norm_rope_append, l_add_rmsnorm};
+    return t;
 }
 
 const LaunchFn* catalog_launchers() {

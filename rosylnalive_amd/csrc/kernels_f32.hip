@@ -38,10 +38,11 @@ constexpr uint32_t kNegZeroPair = 0x80008000u;
 // A block computes a (16 WR TM) x (16 WC TN) tile: WR x WC multiplying waves of TM x TN MFMA tiles, as many staging
 // waves. The loop runs whole groups of D tiles of KS; tiles past k multiply the padding.
 // VEC: x and w 16-byte aligned, k a multiple of 8; otherwise element loads. FULL: k a multiple of D KS, no padding.
+// Up to three weights over one x share a launch, their column tiles side by side: a decode step's q, k and v projections
+// are 64 to 128 chains' worth of blocks each, and one after another each waits its chain out on an idle chip.
 template <int WR, int WC, int TM, int TN, int KS, int D, int NB, bool VEC, bool FULL>
-__global__ __launch_bounds__(128 * WR * WC) void k_matmul_mfma(const float* __restrict__ x,
-                                                               const uint16_t* __restrict__ w, float* __restrict__ y,
-                                                               uint32_t m, uint32_t n, uint32_t k) {
+__global__ __launch_bounds__(128 * WR * WC) void k_matmul_mfma(const float* __restrict__ x, MatmulGroup group,
+                                                               uint32_t m, uint32_t k) {
     constexpr int BM = 16 * WR * TM, BN = 16 * WC * TN, NT = 64 * WR * WC, STEPS = KS / 4, ROW = STEPS + 4;
     constexpr int XR = NT / (KS / 4), WRW = NT / (KS / 8);  // rows staged per pass
     constexpr int XQ = BM / XR, WQ = BN / WRW;              // 16-byte chunks per staging thread
@@ -50,7 +51,11 @@ __global__ __launch_bounds__(128 * WR * WC) void k_matmul_mfma(const float* __re
     static_assert(KS == 64, "chunk maps");
     __shared__ float xs[NB][4 * BM * ROW];
     __shared__ float ws[NB][4 * BN * ROW];
-    const uint32_t i0 = blockIdx.y * BM, j0 = blockIdx.x * BN;
+    uint32_t part = 0, bx = blockIdx.x;
+    while (part + 1 < group.count && bx >= (group.n[part] + BN - 1) / BN) bx -= (group.n[part++] + BN - 1) / BN;
+    const uint16_t* __restrict__ w = group.w[part];
+    float* __restrict__ y = group.y[part];
+    const uint32_t n = group.n[part], i0 = blockIdx.y * BM, j0 = bx * BN;
     if (threadIdx.x >= NT) {
         const uint32_t t = threadIdx.x - NT;
         // chunk q of this thread: x row xr0 + XR q, k 4 xc ..; w row wr0 + WRW q, k 8 wcx ..; the rows a store touches
@@ -218,33 +223,41 @@ __global__ __launch_bounds__(128 * WR * WC) void k_matmul_mfma(const float* __re
 static bool aligned16(const void* p) { return (reinterpret_cast<uintptr_t>(p) & 15u) == 0; }
 
 template <int WR, int WC, int TM, int TN, int KS, int D, int NB>
-static void launch_mfma(bool vec, const float* x, const uint16_t* w, float* y, uint32_t m, uint32_t n, uint32_t k,
-                        hipStream_t s) {
+static void launch_mfma(bool vec, const float* x, const MatmulGroup& g, uint32_t m, uint32_t k, hipStream_t s) {
     constexpr uint32_t BM = 16 * WR * TM, BN = 16 * WC * TN;
-    const dim3 grid((n + BN - 1) / BN, (m + BM - 1) / BM), block(128 * WR * WC);
+    uint32_t tiles = 0;
+    for (uint32_t i = 0; i < g.count; ++i) tiles += (g.n[i] + BN - 1) / BN;
+    const dim3 grid(tiles, (m + BM - 1) / BM), block(128 * WR * WC);
     if (vec && k % (D * KS) == 0 && uint64_t(k) * (BM > BN / 2 ? BM : BN / 2) * 4 < (1ull << 31))
-        hipLaunchKernelGGL((k_matmul_mfma<WR, WC, TM, TN, KS, D, NB, true, true>), grid, block, 0, s, x, w, y, m, n, k);
+        hipLaunchKernelGGL((k_matmul_mfma<WR, WC, TM, TN, KS, D, NB, true, true>), grid, block, 0, s, x, g, m, k);
     else if (vec)
-        hipLaunchKernelGGL((k_matmul_mfma<WR, WC, TM, TN, KS, D, NB, true, false>), grid, block, 0, s, x, w, y, m, n, k);
+        hipLaunchKernelGGL((k_matmul_mfma<WR, WC, TM, TN, KS, D, NB, true, false>), grid, block, 0, s, x, g, m, k);
     else
-        hipLaunchKernelGGL((k_matmul_mfma<WR, WC, TM, TN, KS, D, NB, false, false>), grid, block, 0, s, x, w, y, m, n, k);
+        hipLaunchKernelGGL((k_matmul_mfma<WR, WC, TM, TN, KS, D, NB, false, false>), grid, block, 0, s, x, g, m, k);
 }
 
-void matmul_bf16w(const float* x, const uint16_t* w, float* y, uint32_t m, uint32_t n, uint32_t k, hipStream_t s) {
-    const bool vec = k % 8 == 0 && aligned16(x) && aligned16(w);
+void matmul_bf16w(const float* x, const MatmulGroup& g, uint32_t m, uint32_t k, hipStream_t s) {
+    bool vec = k % 8 == 0 && aligned16(x);
+    uint64_t n = 0, big = 0, small = 0;
+    for (uint32_t i = 0; i < g.count; ++i) {
+        vec = vec && aligned16(g.w[i]);
+        n += g.n[i];
+        big += uint64_t((m + 63) / 64) * ((g.n[i] + 63) / 64);
+        small += uint64_t((m + 31) / 32) * ((g.n[i] + 31) / 32);
+    }
     // Up to 16 rows one MFMA tile per block: an output is one chain however many columns a block has, and two waves find
     // SIMDs of their own (1 x 1024 x 1024: 5.8 us; 32-column blocks 6.0); past 16,384 columns, where the weights' stream
-    // counts, 32 columns (1 x 151,936 x 1024: 79.7 us against 84.1). Above: 32 x 32 tiles (150 x 3072 x 1024: 14.7 us;
-    // 64 x 64 22.1), 64 x 64 from 200 of those tiles on (300 x 3072 x 1024, 240 tiles: 23.2 against 26.3; 2048 x 3072 x
-    // 1024: 126 against 139, 102 TFLOP/s; 300 x 2048 x 1024, 160 tiles: 22.2 against 20.5).
+    // counts, 32 columns (1 x 151,936 x 1024: 79.7 us against 84.1). Above: 32 x 32 tiles, about 26 ns a tile at k 1024
+    // however they fill the chip (480 tiles 14.7 us, 960 26.3, 6144 139), or 64 x 64, 21 us a round of 256 (240 tiles 23.2
+    // us, 480 42.8, 1536 126): the larger where its rounds take less (a round for 800 small tiles).
     if (m <= 16 && n <= 16384)
-        launch_mfma<1, 1, 1, 1, 64, 4, 4>(vec, x, w, y, m, n, k, s);
+        launch_mfma<1, 1, 1, 1, 64, 4, 4>(vec, x, g, m, k, s);
     else if (m <= 16)
-        launch_mfma<1, 2, 1, 1, 64, 8, 4>(vec, x, w, y, m, n, k, s);
-    else if (uint64_t((m + 63) / 64) * ((n + 63) / 64) >= 200)
-        launch_mfma<2, 2, 2, 2, 64, 4, 4>(vec, x, w, y, m, n, k, s);
+        launch_mfma<1, 2, 1, 1, 64, 8, 4>(vec, x, g, m, k, s);
+    else if ((big + 255) / 256 * 800 < small)
+        launch_mfma<2, 2, 2, 2, 64, 4, 4>(vec, x, g, m, k, s);
     else
-        launch_mfma<2, 2, 1, 1, 64, 8, 4>(vec, x, w, y, m, n, k, s);
+        launch_mfma<2, 2, 1, 1, 64, 8, 4>(vec, x, g, m, k, s);
 }
 
 // ---------------------------------------------------------------- attention_gqa_causal

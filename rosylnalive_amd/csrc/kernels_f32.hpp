@@ -8,8 +8,14 @@
 namespace lrm {
 namespace f32k {
 
-// y[m, n] = x[m, k] . w[n, k]^T (bf16 w), every output one ascending fused chain over k.
-void matmul_bf16w(const float* x, const uint16_t* w, float* y, uint32_t m, uint32_t n, uint32_t k, hipStream_t s);
+// y[i][m, n[i]] = x[m, k] . w[i][n[i], k]^T (bf16 w) for i < count, every output one ascending fused chain over k.
+struct MatmulGroup {
+    const uint16_t* w[3];
+    float* y[3];
+    uint32_t n[3];
+    uint32_t count;
+};
+void matmul_bf16w(const float* x, const MatmulGroup& group, uint32_t m, uint32_t k, hipStream_t s);
 
 // attention_gqa_causal on the matrix cores; false (nothing launched) when the shape or an alignment is not covered. A
 // decode row spreads over the chip when `workspace` (kWorkspaceBytes, written by each call, its contents not kept; null:

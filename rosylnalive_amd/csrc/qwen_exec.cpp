@@ -647,6 +647,34 @@ uint32_t QwenExec::forward_fp32(int pos0, int T, float* logits, int lr) {
     const uint32_t LR = uint32_t(c.taps ? T : lr);
     if (LR > dev_.table().row(tk("logits")).count() / V) arg_fail("%u logits rows exceed the logits tensor", LR);
     CommandList* l = dev_.begin();
+    if (!c.taps) {  // the same operations in fewer launches: nobody reads what the separate ones leave between
+        dispatch(l, "embed_gather_bf16", {tk("ids"), tk("model.embed_tokens.weight"), tk("x"), U, H, V});
+        dispatch(l, "rmsnorm_rows", {tk("x"), tk(lname(0, kLayerWeights[0])), tk("h"), U, H, eps});
+        for (int i = 0; i < c.layers; ++i) {
+            const std::string p = "L" + std::to_string(i) + ".";
+            auto w = [&](int k) { return tk(lname(i, kLayerWeights[k])); };
+            const bool last = i + 1 == c.layers;
+            dispatch(l, "matmul_bf16w_triple", {tk("h"), w(1), w(2), w(3), tk("q"), tk("k"), tk("v"), U, QC, KC, KC, H});
+            dispatch(l, "qk_norm_rope_append",
+                     {tk("q"), tk("k"), tk("v"), w(5), w(6), tk("rope.cos"), tk("rope.sin"), tk("qr"), tk(p + "k_cache"),
+                      tk(p + "v_cache"), U, uint32_t(c.heads), uint32_t(c.kv_heads), HD, uint32_t(pos0), eps});
+            dispatch(l, "attention_gqa_causal", {tk("qr"), tk(p + "k_cache"), tk(p + "v_cache"), tk("o"), U, 0,
+                                                 uint32_t(pos0), uint32_t(c.heads), uint32_t(c.kv_heads), HD, scale});
+            dispatch(l, "matmul_bf16w", {tk("o"), w(4), tk("oo"), U, H, QC});
+            dispatch(l, "add_rmsnorm_rows", {tk("x"), tk("oo"), w(7), tk("r"), tk("h2"), U, H, eps});
+            dispatch(l, "matmul_bf16w_pair", {tk("h2"), w(8), w(9), tk("g"), tk("u"), U, I, I, H});
+            dispatch(l, "silu_mul", {tk("g"), tk("u"), tk("d"), U * I});
+            dispatch(l, "matmul_bf16w", {tk("d"), w(10), tk("dd"), U, H, I});
+            dispatch(l, "add_rmsnorm_rows",
+                     {tk("r"), tk("dd"), last ? tk("model.norm.weight") : tk(lname(i + 1, kLayerWeights[0])), tk("x"),
+                      tk(last ? "f" : "h"), U, H, eps});
+            flush(l);
+        }
+        if (LR < U) dispatch(l, "copy_rows", {tk("f"), tk("f_last"), LR, H, U - LR, 0, H, H});
+        dispatch(l, "matmul_bf16w", {tk(LR < U ? "f_last" : "f"), tk("model.embed_tokens.weight"), tk("logits"), LR, V, H});
+        dispatch(l, "argmax_rows", {tk("logits"), tk("argmax"), LR, V});
+        return finish_fp32(l, logits, lr, LR);
+    }
     dispatch(l, "embed_gather_bf16", {tk("ids"), tk("model.embed_tokens.weight"), tk("x"), U, H, V});
     tap_copy(l, "embed.out", tk("x"), T, int(H));
     for (int i = 0; i < c.layers; ++i) {
@@ -717,6 +745,12 @@ uint32_t QwenExec::forward_fp32(int pos0, int T, float* logits, int lr) {
     if (c.taps) tap_copy(l, "logits", tk("logits"), T, int(V));
     l->barrier();
     dispatch(l, "argmax_rows", {tk("logits"), tk("argmax"), LR, V});
+    return finish_fp32(l, logits, lr, LR);
+}
+
+// The last piece, the wait, and the last row's argmax with the requested logits.
+uint32_t QwenExec::finish_fp32(CommandList* l, float* logits, int lr, uint32_t LR) {
+    const uint32_t V = cfg_.vocab;
     pieces_.push_back(dev_.submit(l));
     dev_.release(l);
     dev_.collect(false, static_cast<const uint32_t*>(ptr("argmax")) + (LR - 1), nullptr, nullptr, 0);

@@ -99,6 +99,7 @@ class QwenExec {
     void plan();
     void upload_rope(const uint32_t* inv_freq_bits);
     uint32_t forward_fp32(int pos0, int t, float* logits, int logits_rows);
+    uint32_t finish_fp32(CommandList* l, float* logits, int logits_rows, uint32_t rows);
     uint32_t forward_fast(int seq, int pos0, int t, float* logits, int logits_rows);
     // bits: the fp16 range sites of all chunks
     uint32_t forward_chunks(int seq, int pos0, const int32_t* ids, int t, float* logits, int logits_rows, uint32_t& bits);
