@@ -245,11 +245,10 @@ struct GemmStampEnd {  // the epilogue's end, at whichever return the lane leave
 // tiles go through two register sets into two padded LDS buffers with every load two k steps ahead.
 template <int EPI, int BN, bool DMA, int BM = GBM>
 __global__ __launch_bounds__(256, 2) void k_gemm(GemmArgs p) {
-    static_assert(BN == 128 || (BN == 64 && (EPI == EPI_F32 || EPI == EPI_RESID || EPI == EPI_PART)) ||
-                      (BN == 192 && EPI == EPI_SWIGLU && DMA),
-                  "QKV takes 128 columns, SwiGLU 128 or 192 (64 or 96 gate / up pairs)");
-    static_assert(BM == GBM || (BM == 64 && (EPI == EPI_QKV || EPI == EPI_PART) && !DMA),
-                  "64-row tiles: the q|k|v and k-split register loops only");
+    static_assert(BN == 128 || (BN == 64 && EPI != EPI_QKV && (EPI != EPI_SWIGLU || BM == 64)) ||
+                      (BN == 32 && EPI == EPI_PART && BM == 64) || (BN == 192 && EPI == EPI_SWIGLU && DMA),
+                  "QKV takes 128 columns, SwiGLU 64 (64 rows), 128 or 192 (32, 64 or 96 gate / up pairs)");
+    static_assert(BM == GBM || (BM == 64 && EPI != EPI_RESID && !DMA), "64-row tiles: register loops only");
     constexpr int MI = BM / 32;   // MFMA row tiles per wave: each wave owns BM / 2 rows
     constexpr int PAIR = BN / 2;  // SWIGLU: gate / up pairs per tile
     // the k range of this block: all of k, or split z of a PART launch (A and W then start kz columns in)
@@ -693,7 +692,7 @@ __global__ __launch_bounds__(256, 2) void k_gemm(GemmArgs p) {
         __syncthreads();
         uint32_t bad = 0;
 #pragma unroll
-        for (int k = 0; k < CH / 2; ++k) {  // 128 rows x CH chunks = 256 (CH / 2) chunks
+        for (int k = 0; k < BM * CH / 256; ++k) {  // BM rows x CH chunks, 256 at a time
             const int q = t + 256 * k, row = q / CH, ch = q % CH, m = m0 + row, col = tx * PAIR + ch * 8;
             if (m >= p.M || col >= p.inter) continue;
             const u32x4 v = *reinterpret_cast<const u32x4*>(As + row * AR + ch * 8);
@@ -2153,19 +2152,34 @@ static GemmArgs gemm_base(void* const* p, uint32_t m, uint32_t n, uint32_t k) {
     return a;
 }
 
-// 15 gemm_qkv_rope: h, w, q_norm, k_norm, cos, sin, q, k_cache, v_cache, m, hidden, q_heads, kv_heads, pos0, max_pos,
-// The GEMM's direct-to-LDS loop needs two blocks on every CU (MI355X: 256 CUs, two 64 KiB blocks each) for the whole
-// launch: grids of whole rounds of 512 tiles, or long enough (4 rounds) that a last partial round hardly counts. In a
-// partial round a CU holds one block, which the register-pipelined loop (loads two k steps ahead) serves better
-// (measured: the 768-tile SwiGLU GEMM of a 2048-token prefill, 42 against 44 us).
+// The GEMM's direct-to-LDS loop needs two blocks on every CU (MI355X: 256 CUs, two 64 KiB blocks each) for most of the
+// launch: rounds of 512 tiles at least three quarters full, or so many (4) that a partial last one hardly counts. In an
+// emptier round a CU holds one block, which the register-pipelined loop (loads two k steps ahead) serves better (measured:
+// the 768-tile SwiGLU GEMM of a 2048-token prefill, 42 against 44 us). Four layers, device time, against whole rounds only:
+// 0.6B shape at 1000 rows (384 SwiGLU tiles) 437 -> 423 us, 1800 (480 q|k|v tiles) 625 -> 609; 1.7B at 600 641 -> 625.
+static bool mostly_full(uint64_t tiles) { return tiles * 4 >= (tiles + 511) / 512 * (512 * 3); }
 static bool two_per_cu(const dim3& g) {
     const uint64_t tiles = uint64_t(g.x) * g.y;
-    return tiles >= 512 && (tiles % 512 == 0 || tiles >= 4 * 512);
+    return mostly_full(tiles) || tiles >= 4 * 512;
 }
-// q|k|v tiles of 64 rows where 128-row tiles leave CUs without a tile (512 rows: 32 x 4 tiles on half the CUs, 32 x 8
-// on all of them; the 512-token forward 2.40-2.41 -> 2.27 ms)
-static bool qkv_rows64(uint32_t m, uint32_t heads) { return m > 64 && uint64_t(heads) * ((m + 127) / 128) < 256; }
+// The register loop's tile: 128 rows (0), 64 rows (1), or 64 rows and half the columns (2; `half` 0: no such form). Smaller
+// tiles reach more CUs and waste fewer rows past m, but a round of 256 (one per CU; the loop waits for its loads more than
+// it multiplies) of them takes 0.63 / 0.5 of a round of the largest: the fewest such units win, the larger tile on a tie.
+// Four layers, device time, against 128 rows up to 64 rows and 64 from there to 256 tiles: 0.6B shape at 37 rows 284 -> 195
+// us, 100 253 -> 207, 256 267 -> 230; 1.7B at 37 412 -> 314, 100 386 -> 339. The sums' order does not depend on the tile.
+static int small_tile(uint64_t full, uint64_t rows64, uint64_t half) {
+    auto rounds = [](uint64_t tiles) { return (tiles + 255) / 256; };
+    const uint64_t a = rounds(full) * 100, b = rounds(rows64) * 63, c = half ? rounds(half) * 50 : ~uint64_t(0);
+    return a <= b && a <= c ? 0 : b <= c ? 1 : 2;
+}
+static uint64_t tiles_of(uint64_t m, uint64_t rows, uint64_t n, uint64_t cols) {
+    return ((m + rows - 1) / rows) * ((n + cols - 1) / cols);
+}
+static bool qkv_rows64(uint32_t m, uint32_t heads) {
+    return small_tile(tiles_of(m, 128, heads, 1), tiles_of(m, 64, heads, 1), 0) == 1;
+}
 
+// 15 gemm_qkv_rope: h, w, q_norm, k_norm, cos, sin, q, k_cache, v_cache, m, hidden, q_heads, kv_heads, pos0, max_pos,
 // eps
 static void l_gemm_qkv(const PreparedDispatch& pd, void* const* p, hipStream_t s) {
     const uint32_t* w = pd.words.data();
@@ -2220,16 +2234,22 @@ static void l_gemm_resid(const PreparedDispatch& pd, void* const* p, hipStream_t
                            s, a);
 }
 
-// gemm_swiglu's gate / up pairs per tile: 96 where that makes whole rounds of 512 tiles for the direct-to-LDS loop
-// (Qwen3-0.6B at 2048 rows: 32 x 16 tiles, where 64 pairs give 768 tiles, one and a half rounds); else 64
-static int swiglu_pairs(uint32_t m, uint32_t inter) {
-    const uint64_t rows = (m + GBM - 1) / GBM;
-    if (inter % 96 == 0 && (uint64_t(inter / 96) * rows) % 512 == 0) return 96;
-    return 64;
+// gemm_swiglu's tile: 96 gate / up pairs of 128 rows where that mostly fills rounds of 512 tiles for the direct-to-LDS loop
+// (the 0.6B shape at 2048 rows: 32 x 16 tiles, where 64 pairs give one and a half rounds; at 1500 rows 384 tiles: four
+// layers 575 -> 550 us; 1.7B at 777, 448 tiles: 769 -> 736), else 64 pairs where those do, else the register loop's tile.
+struct SwigluTile {
+    uint32_t pairs, rows;
+    bool dma;
+};
+static SwigluTile swiglu_tile(uint32_t m, uint32_t inter) {
+    if (inter % 96 == 0 && mostly_full(tiles_of(m, 128, inter, 96))) return {96, 128, true};
+    if (two_per_cu(dim3((inter + 63) / 64, (m + 127) / 128))) return {64, 128, true};
+    const int t = small_tile(tiles_of(m, 128, inter, 64), tiles_of(m, 64, inter, 64), tiles_of(m, 64, inter, 32));
+    return {t == 2 ? 32u : 64u, t ? 64u : 128u, false};
 }
 static dim3 swiglu_grid(uint32_t m, uint32_t inter) {
-    const uint32_t pairs = uint32_t(swiglu_pairs(m, inter));
-    return dim3((inter + pairs - 1) / pairs, (m + GBM - 1) / GBM);
+    const SwigluTile t = swiglu_tile(m, inter);
+    return dim3((inter + t.pairs - 1) / t.pairs, (m + t.rows - 1) / t.rows);
 }
 
 // 18 gemm_swiglu: a, w (2 inter rows), y, m, inter, k, a_shift
@@ -2240,23 +2260,44 @@ static void l_gemm_swiglu(const PreparedDispatch& pd, void* const* p, hipStream_
     a.inter = int(w[5]);
     a.ascale = a_scale(w[7]);
     const dim3 grid = swiglu_grid(w[4], w[5]);
-    const int pairs = swiglu_pairs(w[4], w[5]);
-    if (pairs == 96)
+    const SwigluTile t = swiglu_tile(w[4], w[5]);
+    if (t.pairs == 96)
         hipLaunchKernelGGL((k_gemm<EPI_SWIGLU, 192, true>), grid, dim3(256), 0, s, a);
-    else if (two_per_cu(grid))
+    else if (t.dma)
         hipLaunchKernelGGL((k_gemm<EPI_SWIGLU, 128, true>), grid, dim3(256), 0, s, a);
+    else if (t.pairs == 32)
+        hipLaunchKernelGGL((k_gemm<EPI_SWIGLU, 64, false, 64>), grid, dim3(256), 0, s, a);
+    else if (t.rows == 64)
+        hipLaunchKernelGGL((k_gemm<EPI_SWIGLU, 128, false, 64>), grid, dim3(256), 0, s, a);
     else
         hipLaunchKernelGGL((k_gemm<EPI_SWIGLU, 128, false>), grid, dim3(256), 0, s, a);
 }
 
+// gemm_f32's tile: 128 columns, 64 in the register loop's smallest form
+static bool f32_dma(uint32_t m, uint32_t n) {
+    const uint64_t tiles = tiles_of(m, 128, n, 128);
+    return tiles >= 512 && (tiles % 512 == 0 || tiles >= 4 * 512);
+}
+static int f32_tile(uint32_t m, uint32_t n) {
+    return f32_dma(m, n) ? 0 : small_tile(tiles_of(m, 128, n, 128), tiles_of(m, 64, n, 128), tiles_of(m, 64, n, 64));
+}
+static dim3 f32_grid(uint32_t m, uint32_t n) {
+    const int t = f32_tile(m, n);
+    return dim3(t == 2 ? (n + 63) / 64 : (n + 127) / 128, t ? (m + 63) / 64 : (m + 127) / 128);
+}
 // 19 gemm_f32: a, w, y, m, n, k
 static void l_gemm_f32(const PreparedDispatch& pd, void* const* p, hipStream_t s) {
     const uint32_t* w = pd.words.data();
     GemmArgs a = gemm_base(p, w[4], w[5], w[6]);
     a.y32 = (float*)p[2];
-    const dim3 grid((w[5] + GBN - 1) / GBN, (w[4] + GBM - 1) / GBM);
-    if (two_per_cu(grid))
+    const dim3 grid = f32_grid(w[4], w[5]);
+    const int t = f32_tile(w[4], w[5]);
+    if (f32_dma(w[4], w[5]))
         hipLaunchKernelGGL((k_gemm<EPI_F32, 128, true>), grid, dim3(256), 0, s, a);
+    else if (t == 2)
+        hipLaunchKernelGGL((k_gemm<EPI_F32, 64, false, 64>), grid, dim3(256), 0, s, a);
+    else if (t == 1)
+        hipLaunchKernelGGL((k_gemm<EPI_F32, 128, false, 64>), grid, dim3(256), 0, s, a);
     else
         hipLaunchKernelGGL((k_gemm<EPI_F32, 128, false>), grid, dim3(256), 0, s, a);
 }
@@ -2493,8 +2534,17 @@ static void l_prefetch(const PreparedDispatch& pd, void* const* p, hipStream_t s
 static bool resid_split_skinny(uint32_t m, uint32_t k, uint32_t splits) {
     return m <= 16 && (k / splits) % (kSkWaves * 128) == 0;
 }
-// 64-row tiles for grids of 128 x 64 tiles under one block per CU
-static bool resid_rows64(uint32_t m, uint64_t blocks128) { return m > 64 && blocks128 < 256; }
+// its tile: 128 x 64 on the direct-to-LDS loop (-1; four layers at 777 rows of the 0.6B shape, 448 tiles: 411 -> 399 us) or
+// the register loop's 128 x 64 (0), 64 x 64 (1) or 64 x 32 (2)
+static int resid_tile(uint32_t m, uint32_t n, uint32_t splits) {
+    const uint64_t full = tiles_of(m, 128, n, 64) * splits;
+    if (mostly_full(full)) return -1;
+    return small_tile(full, tiles_of(m, 64, n, 64) * splits, tiles_of(m, 64, n, 32) * splits);
+}
+static dim3 resid_grid(uint32_t m, uint32_t n, uint32_t splits) {
+    const int t = resid_tile(m, n, splits);
+    return dim3(t == 2 ? (n + 31) / 32 : (n + 63) / 64, t > 0 ? (m + 63) / 64 : (m + 127) / 128, splits);
+}
 static void l_gemm_resid_split(const PreparedDispatch& pd, void* const* p, hipStream_t s) {
     const uint32_t* w = pd.words.data();
     if (resid_split_skinny(w[4], w[6], w[7])) {
@@ -2507,15 +2557,13 @@ static void l_gemm_resid_split(const PreparedDispatch& pd, void* const* p, hipSt
     a.y32 = (float*)p[2];
     a.ksplit = int(w[6] / w[7]);
     a.ascale = a_unscale(w[8]);
-    const dim3 grid((w[5] + 63) / 64, (w[4] + GBM - 1) / GBM, w[7]);
-    const uint64_t blocks = uint64_t(grid.x) * grid.y * grid.z;
-    if (blocks % 512 == 0)  // whole rounds of two blocks per CU: the direct-to-LDS loop
-        hipLaunchKernelGGL((k_gemm<EPI_PART, 64, true>), grid, dim3(256), 0, s, a);
-    else if (resid_rows64(w[4], blocks))  // 64-row tiles, twice the blocks
-        hipLaunchKernelGGL((k_gemm<EPI_PART, 64, false, 64>), dim3(grid.x, (w[4] + 63) / 64, grid.z), dim3(256), 0, s,
-                           a);
-    else
-        hipLaunchKernelGGL((k_gemm<EPI_PART, 64, false>), grid, dim3(256), 0, s, a);
+    const dim3 grid = resid_grid(w[4], w[5], w[7]);
+    switch (resid_tile(w[4], w[5], w[7])) {
+        case -1: hipLaunchKernelGGL((k_gemm<EPI_PART, 64, true>), grid, dim3(256), 0, s, a); break;
+        case 0: hipLaunchKernelGGL((k_gemm<EPI_PART, 64, false>), grid, dim3(256), 0, s, a); break;
+        case 1: hipLaunchKernelGGL((k_gemm<EPI_PART, 64, false, 64>), grid, dim3(256), 0, s, a); break;
+        default: hipLaunchKernelGGL((k_gemm<EPI_PART, 32, false, 64>), grid, dim3(256), 0, s, a); break;
+    }
 }
 
 // 40 residual_add_norm: x, partials, w, y, rows, cols, splits, eps
@@ -2708,7 +2756,10 @@ std::vector<KernelSpec> fast_catalog() {
                  }});
     // 19 gemm_f32: a, w, y, m, n, k
     c.push_back({"gemm_f32", "fast", {256, 1, 1}, false,
-                 [](const uint32_t* w) { return Grid3{(int64_t(w[5]) + 127) / 128, (int64_t(w[4]) + 127) / 128, 1}; },
+                 [](const uint32_t* w) {
+                     const dim3 g = f32_grid(w[4], w[5]);
+                     return Grid3{g.x, g.y, 1};
+                 },
                  {TOK_R("a", DT(F16)), TOK_R("w", DT(F16)), TOK_W("y", DT(F32)), U32F("m"), U32F("n"), U32F("k")},
                  [](const uint32_t* w, const uint32_t* c) {
                      if (w[6] % 64 || w[6] < 64) contract_fail("gemm_f32: k must be a positive multiple of 64");
@@ -2942,9 +2993,8 @@ std::vector<KernelSpec> fast_catalog() {
     c.push_back({"gemm_residual_split", "fast", {256, 1, 1}, false,
                  [](const uint32_t* w) {
                      if (resid_split_skinny(w[4], w[6], w[7])) return Grid3{(int64_t(w[5]) + 15) / 16, w[7], 1};
-                     const int64_t gx = (int64_t(w[5]) + 63) / 64, g128 = (int64_t(w[4]) + 127) / 128;
-                     const int64_t rows = resid_rows64(w[4], uint64_t(gx * g128 * w[7])) ? 64 : 128;
-                     return Grid3{gx, (int64_t(w[4]) + rows - 1) / rows, w[7]};
+                     const dim3 g = resid_grid(w[4], w[5], w[7]);
+                     return Grid3{g.x, g.y, g.z};
                  },
                  {TOK_R("a", DT(F16)), TOK_R("w", DT(F16)), TOK_W("partials", DT(F32)), U32F("m"), U32F("n"), U32F("k"),
                   U32F("splits"), U32F("a_shift")},
