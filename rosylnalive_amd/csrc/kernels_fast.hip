@@ -1276,6 +1276,22 @@ __device__ __forceinline__ void load_chunks_16(const uint16_t* row, int K, uint4
     }
 }
 
+// The same with non-temporal loads, for weight rows that one wave reads once per step.
+template <int NCH>
+__device__ __forceinline__ void load_chunks_stream(const uint16_t* row, int K, uint4 (&w)[NCH]) {
+    typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
+    const int lane = threadIdx.x & 63;
+#pragma unroll
+    for (int c = 0; c < NCH; ++c) {
+        const int k0 = 512 * c + 8 * lane;
+        w[c] = make_uint4(0, 0, 0, 0);
+        if (k0 < K) {
+            const u32x4 t = __builtin_nontemporal_load(reinterpret_cast<const u32x4*>(row + k0));
+            w[c] = make_uint4(t.x, t.y, t.z, t.w);
+        }
+    }
+}
+
 // v <- widen(nw) * (v * r), r = 1 / sqrt(sum(v^2) / K + eps): the RMSNorm of the whole vector (padding lanes hold 0).
 template <int NCH>
 __device__ __forceinline__ void rmsnorm_chunks(float (&v)[NCH][8], const uint4 (&nw)[NCH], int K, float eps) {
@@ -1310,19 +1326,26 @@ __device__ __forceinline__ float dot_chunks(const uint4 (&w)[NCH], const float (
 }
 
 // ---------------------------------------------------------------- 20 gemv_norm_dec: y[n] = w[n] . RMSNorm(x)
-template <int NCH>
+// R rows per wave (1 or 2, launcher's rule): the vector and its norm are loaded and computed once for the R rows, each
+// row's own sums unchanged. Bound by the weight stream; at one row per wave it reads 8 KB of x and 4 KB of norm (cache
+// hits, but loads in flight all the same) for 4 KB of weights at K 2048.
+template <int NCH, int R>
 __global__ __launch_bounds__(256) void k_gemv_norm_dec(const float* x, const uint16_t* nw, const uint16_t* w, float* y,
                                                        int n, int k, float eps) {
-    const int row = blockIdx.x * 4 + (threadIdx.x >> 6);
+    const int row = (blockIdx.x * 4 + (threadIdx.x >> 6)) * R;
     if (row >= n) return;
-    uint4 wv[NCH], g[NCH];
+    uint4 wv[R][NCH], g[NCH];
     float xv[NCH][8];
-    load_chunks_16<NCH>(w + size_t(row) * k, k, wv);
+#pragma unroll
+    for (int r = 0; r < R; ++r) load_chunks_stream<NCH>(w + size_t(min(row + r, n - 1)) * k, k, wv[r]);
     load_chunks_f32<NCH>(x, k, xv);
     load_chunks_16<NCH>(nw, k, g);
     rmsnorm_chunks<NCH>(xv, g, k, eps);
-    const float out = dot_chunks<NCH>(wv, xv);
-    if ((threadIdx.x & 63) == 0) y[row] = out;
+#pragma unroll
+    for (int r = 0; r < R; ++r) {
+        const float out = dot_chunks<NCH>(wv[r], xv);
+        if ((threadIdx.x & 63) == 0 && row + r < n) y[row + r] = out;
+    }
 }
 
 // ---------------------------------------------------------------- 21 attention_decode_f16
@@ -1683,21 +1706,29 @@ __global__ __launch_bounds__(256) void k_gemv_resid_dec(const float* a, const ui
 }
 
 // ---------------------------------------------------------------- 24 gemv_swiglu_dec: a[j] = silu(g_j . h) * (u_j . h)
-template <int NCH>
+// R gate/up pairs per wave, as 20 gemv_norm_dec.
+template <int NCH, int R>
 __global__ __launch_bounds__(256) void k_gemv_swiglu_dec(const float* x, const uint16_t* nw, const uint16_t* w,
                                                          float* y, int inter, int hidden, float eps) {
-    const int j = blockIdx.x * 4 + (threadIdx.x >> 6);
+    const int j = (blockIdx.x * 4 + (threadIdx.x >> 6)) * R;
     if (j >= inter) return;
-    uint4 wg[NCH], wu[NCH], g[NCH];
+    uint4 wg[R][NCH], wu[R][NCH], g[NCH];
     float xv[NCH][8];
-    load_chunks_16<NCH>(w + size_t(j) * hidden, hidden, wg);
-    load_chunks_16<NCH>(w + size_t(inter + j) * hidden, hidden, wu);
+#pragma unroll
+    for (int r = 0; r < R; ++r) {
+        const size_t jr = size_t(min(j + r, inter - 1));
+        load_chunks_stream<NCH>(w + jr * hidden, hidden, wg[r]);
+        load_chunks_stream<NCH>(w + (size_t(inter) + jr) * hidden, hidden, wu[r]);
+    }
     load_chunks_f32<NCH>(x, hidden, xv);
     load_chunks_16<NCH>(nw, hidden, g);
     rmsnorm_chunks<NCH>(xv, g, hidden, eps);
-    const float gv = dot_chunks<NCH>(wg, xv);
-    const float uv = dot_chunks<NCH>(wu, xv);
-    if ((threadIdx.x & 63) == 0) y[j] = gv / (1.0f + __expf(-gv)) * uv;
+#pragma unroll
+    for (int r = 0; r < R; ++r) {
+        const float gv = dot_chunks<NCH>(wg[r], xv);
+        const float uv = dot_chunks<NCH>(wu[r], xv);
+        if ((threadIdx.x & 63) == 0 && j + r < inter) y[j + r] = gv / (1.0f + __expf(-gv)) * uv;
+    }
 }
 
 // ---------------------------------------------------------------- 25 lmhead_dec
@@ -2302,7 +2333,20 @@ static void l_gemm_f32(const PreparedDispatch& pd, void* const* p, hipStream_t s
         hipLaunchKernelGGL((k_gemm<EPI_F32, 128, false>), grid, dim3(256), 0, s, a);
 }
 
-// The decode GEMVs: one row (or gate/up pair) per wave, 4 waves per block; NCH, the 512-wide k-chunks per lane, is
+// Rows (or gate/up pairs) per wave of the two normed GEMVs: two where that still gives each CU two blocks of four
+// waves, for a vector of at most 2048 (the register room). One wave of a CU's SIMD with twice the loads in flight
+// streams as well as two, and half as many waves load and norm the vector. Measured with the non-temporal weight loads,
+// in a step that streams 800 MB: 12.9 -> 11.8 us for 2 x 6144 rows of 2048 (50 MB), 6.3 -> 5.8 for 4096 rows of 2048;
+// four rows 12.7 and 5.6. The residual GEMVs (2048 rows) gain nothing from either: 7.2 / 4.3 us as they are,
+// 7.2 / 4.5 with both. A whole step at that layer: 6 layers 261 -> 238 us, 4 layers 181 -> 169; with 2 layers, whose 200 MB
+// of weights the last-level cache would have kept, 95 -> 97.
+static int gemv_rows(uint32_t rows, uint32_t k) { return rows >= 4096 && k <= 2048 ? 2 : 1; }
+static uint32_t gemv_norm_blocks(uint32_t rows, uint32_t k) {
+    const uint32_t per = 4u * uint32_t(gemv_rows(rows, k));
+    return (rows + per - 1) / per;
+}
+
+// The decode GEMVs: one row (or gate/up pair) per wave unless said otherwise, 4 waves per block; NCH, the 512-wide k-chunks per lane, is
 // rounded up to one of the compiled widths.
 static uint32_t gemv_blocks(uint32_t rows) { return (rows + 3) / 4; }
 static int nch_bucket(uint32_t k) {
@@ -2327,8 +2371,10 @@ static int nch_bucket(uint32_t k) {
 // 20 gemv_norm_dec: x, norm, w, y, n, k, eps
 static void l_gemv_norm(const PreparedDispatch& pd, void* const* p, hipStream_t s) {
     const uint32_t* w = pd.words.data();
+    const bool two = gemv_rows(w[5], w[6]) == 2;
 #define L_NORM(N)                                                                                                    \
-    hipLaunchKernelGGL(k_gemv_norm_dec<N>, dim3(gemv_blocks(w[5])), dim3(256), 0, s, (const float*)p[0],            \
+    hipLaunchKernelGGL((two && N <= 4 ? k_gemv_norm_dec<N, (N <= 4 ? 2 : 1)> : k_gemv_norm_dec<N, 1>),               \
+                       dim3(gemv_norm_blocks(w[5], w[6])), dim3(256), 0, s, (const float*)p[0],                      \
                        (const uint16_t*)p[1], (const uint16_t*)p[2], (float*)p[3], int(w[5]), int(w[6]), f32_of(w[7]))
     NCH_DISPATCH(w[6], L_NORM)
 #undef L_NORM
@@ -2418,8 +2464,10 @@ static void l_gemv_resid(const PreparedDispatch& pd, void* const* p, hipStream_t
 // 24 gemv_swiglu_dec: x, norm, w, y, inter, hidden, eps
 static void l_gemv_swiglu(const PreparedDispatch& pd, void* const* p, hipStream_t s) {
     const uint32_t* w = pd.words.data();
+    const bool two = gemv_rows(w[5], w[6]) == 2;
 #define L_SWIGLU(N)                                                                                                  \
-    hipLaunchKernelGGL(k_gemv_swiglu_dec<N>, dim3(gemv_blocks(w[5])), dim3(256), 0, s, (const float*)p[0],          \
+    hipLaunchKernelGGL((two && N <= 4 ? k_gemv_swiglu_dec<N, (N <= 4 ? 2 : 1)> : k_gemv_swiglu_dec<N, 1>),           \
+                       dim3(gemv_norm_blocks(w[5], w[6])), dim3(256), 0, s, (const float*)p[0],                      \
                        (const uint16_t*)p[1], (const uint16_t*)p[2], (float*)p[3], int(w[5]), int(w[6]), f32_of(w[7]))
     NCH_DISPATCH(w[6], L_SWIGLU)
 #undef L_SWIGLU
@@ -2769,7 +2817,7 @@ std::vector<KernelSpec> fast_catalog() {
                  }});
     // 20 gemv_norm_dec: x, norm, w, y, n, k, eps
     c.push_back({"gemv_norm_dec", "fast", {256, 1, 1}, true,
-                 [](const uint32_t* w) { return Grid3{gemv_blocks(w[5]), 1, 1}; },
+                 [](const uint32_t* w) { return Grid3{gemv_norm_blocks(w[5], w[6]), 1, 1}; },
                  {TOK_R("x", DT(F32)), TOK_R("norm", DT(BF16)), TOK_R("w", DT(BF16)), TOK_W("y", DT(F32)), U32F("n"),
                   U32F("k"), F32F("eps")},
                  [](const uint32_t* w, const uint32_t* c) {
@@ -2824,7 +2872,7 @@ std::vector<KernelSpec> fast_catalog() {
                  }});
     // 24 gemv_swiglu_dec: x, norm, w, y, inter, hidden, eps
     c.push_back({"gemv_swiglu_dec", "fast", {256, 1, 1}, true,
-                 [](const uint32_t* w) { return Grid3{gemv_blocks(w[5]), 1, 1}; },
+                 [](const uint32_t* w) { return Grid3{gemv_norm_blocks(w[5], w[6]), 1, 1}; },
                  {TOK_R("x", DT(F32)), TOK_R("norm", DT(BF16)), TOK_R("w", DT(BF16)), TOK_W("y", DT(F32)),
                   U32F("inter"), U32F("hidden"), F32F("eps")},
                  [](const uint32_t* w, const uint32_t* c) {
