@@ -2,7 +2,7 @@
 //   - heap constants, arenas and HeapLayout / HeapPlanner   (src/Lrm.Gpu.Core/HeapLayout.fs:149-525)
 //   - the 64-byte TensorRow and the sealed TensorTable image (src/Lrm.Gpu.Core/TensorTable.fs:46-474)
 //   - the 128-byte ArgBlock, catalog grids and folding        (src/Lrm.Gpu.Core/ArgBlock.fs:240-393)
-//   - the kernel catalog (ids 0..13 as catalog.json, plus the appended bf16 kernels of this backend)
+//   - the kernel catalog (ids 0..13 as catalog.json, plus this backend's appended fast and fused fp32 kernels)
 //   - Dispatch.prepare: word rules, token rules, aliasing     (src/Lrm.Gpu.Core/Dispatch.fs:48-173)
 // Violations throw ContractError, the counterpart of GpuContractException (src/Lrm.Gpu.Core/Errors.fs:7-13).
 #pragma once

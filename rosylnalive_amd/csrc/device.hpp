@@ -164,8 +164,9 @@ class Device {
 
     // IKernelSet. Two kernel sets, each its own ExecutionClass (its own shader-set hash), since they make different
     // bit-identity claims:
-    //   Reference: the reference's catalog, ids 0 .. fast_first_id() - 1, which keeps the BatchInvariance contract
-    //     (a row alone equals the row in any batch; prefill equals decode and any chunked prefill);
+    //   Reference: the reference's catalog, ids 0 .. fast_first_id() - 1, and the fused fp32 kernels, ids kFusedFirstId and
+    //     up, which keeps the BatchInvariance contract (a row alone equals the row in any batch; prefill equals decode and
+    //     any chunked prefill);
     //   Fast: every id (the reference's catalog and the fast path), which only claims that the same work on the same
     //     inputs gives the same bits: its k-split and attention-split choices depend on the row count, and its
     //     prefill and decode kernels sum in different orders.

@@ -2346,8 +2346,8 @@ static uint32_t gemv_norm_blocks(uint32_t rows, uint32_t k) {
     return (rows + per - 1) / per;
 }
 
-// The decode GEMVs: one row (or gate/up pair) per wave unless said otherwise, 4 waves per block; NCH, the 512-wide k-chunks per lane, is
-// rounded up to one of the compiled widths.
+// The decode GEMVs: one row (or gate/up pair) per wave where no rule says two, 4 waves per block; NCH, the 512-wide
+// k-chunks per lane, is rounded up to one of the compiled widths.
 static uint32_t gemv_blocks(uint32_t rows) { return (rows + 3) / 4; }
 static int nch_bucket(uint32_t k) {
     const uint32_t c = (k + 511) / 512;

@@ -5,8 +5,8 @@
   padding past k must keep a chain's -0).
 - attention_gqa_causal: the matrix-core kernel (16-byte aligned tensors, head_dim 16, 32, 64, 128) equals the general
   kernel, which the same tensors one float off their alignment take, bit for bit: one wave per tile and eight, tiles that
-  end inside a row's heads, block edges, the single query row's three launches (up to and past their workspace), and an infinity or NaN among the values of keys past a query's own, which only
-  the queries that own them may see.
+  end inside a row's heads, block edges, the single query row's three launches (up to and past their workspace), and an infinity or NaN among the
+  values of keys past a query's own, which only the queries that own them may see.
 """
 import numpy as np
 import pytest
@@ -72,7 +72,8 @@ def _attention(q, k, v, qh, kvh, hd, past, shift):
 @pytest.mark.parametrize("rows,past,qh,kvh,hd,odd", [
     (1, 0, 4, 2, 16, False), (1, 56, 4, 2, 16, False), (17, 47, 6, 2, 32, False), (5, 59, 8, 1, 64, False),
     (1, 63, 16, 8, 128, False), (1, 700, 16, 8, 128, False), (1, 64, 4, 4, 128, False), (1, 5000, 8, 2, 64, False),
-    (1, 511, 4, 2, 16, False), (1, 448, 4, 1, 32, False), (1, 21500, 16, 8, 128, False), (150, 0, 16, 8, 128, False), (9, 1015, 16, 8, 128, False),
+    (1, 511, 4, 2, 16, False), (1, 448, 4, 1, 32, False), (1, 21500, 16, 8, 128, False), (150, 0, 16, 8, 128, False),
+    (9, 1015, 16, 8, 128, False), (1030, 0, 16, 8, 128, False),
     (1030, 0, 64, 32, 16, False), (270, 3, 512, 128, 32, False), (70, 30, 4, 2, 64, True), (40, 500, 16, 8, 128, True),
     (1030, 5, 64, 32, 16, True)])
 def test_attention_equals_the_general_kernel(rows, past, qh, kvh, hd, odd):
