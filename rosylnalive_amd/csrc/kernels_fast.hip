@@ -1326,25 +1326,42 @@ __device__ __forceinline__ float dot_chunks(const uint4 (&w)[NCH], const float (
 }
 
 // ---------------------------------------------------------------- 20 gemv_norm_dec: y[n] = w[n] . RMSNorm(x)
-// R rows per wave (1 or 2, launcher's rule): the vector and its norm are loaded and computed once for the R rows, each
-// row's own sums unchanged. Bound by the weight stream; at one row per wave it reads 8 KB of x and 4 KB of norm (cache
-// hits, but loads in flight all the same) for 4 KB of weights at K 2048.
-template <int NCH, int R>
+template <int NCH>
 __global__ __launch_bounds__(256) void k_gemv_norm_dec(const float* x, const uint16_t* nw, const uint16_t* w, float* y,
                                                        int n, int k, float eps) {
-    const int row = (blockIdx.x * 4 + (threadIdx.x >> 6)) * R;
+    const int row = blockIdx.x * 4 + (threadIdx.x >> 6);
     if (row >= n) return;
-    uint4 wv[R][NCH], g[NCH];
+    uint4 wv[NCH], g[NCH];
     float xv[NCH][8];
-#pragma unroll
-    for (int r = 0; r < R; ++r) load_chunks_stream<NCH>(w + size_t(min(row + r, n - 1)) * k, k, wv[r]);
+    load_chunks_16<NCH>(w + size_t(row) * k, k, wv);
     load_chunks_f32<NCH>(x, k, xv);
     load_chunks_16<NCH>(nw, k, g);
     rmsnorm_chunks<NCH>(xv, g, k, eps);
-#pragma unroll
-    for (int r = 0; r < R; ++r) {
-        const float out = dot_chunks<NCH>(wv[r], xv);
-        if ((threadIdx.x & 63) == 0 && row + r < n) y[row + r] = out;
+    const float out = dot_chunks<NCH>(wv, xv);
+    if ((threadIdx.x & 63) == 0) y[row] = out;
+}
+
+// Two rows per wave (gemv_rows below): the vector and its norm are loaded and computed once for both, each row's own sums
+// unchanged. Bound by the weight stream; at one row per wave it reads 8 KB of x and 4 KB of norm (cache hits, but loads in
+// flight all the same) for 4 KB of weights at K 2048. Its own kernel: with the row count a parameter of one kernel the
+// one-row form compiled to other load orders and the 0.6B shape's 28-layer list took 761 us a step instead of 736.
+template <int NCH>
+__global__ __launch_bounds__(256) void k_gemv_norm_dec2(const float* x, const uint16_t* nw, const uint16_t* w, float* y,
+                                                        int n, int k, float eps) {
+    const int row = (blockIdx.x * 4 + (threadIdx.x >> 6)) * 2;
+    if (row >= n) return;
+    const int row1 = min(row + 1, n - 1);
+    uint4 w0[NCH], w1[NCH], g[NCH];
+    float xv[NCH][8];
+    load_chunks_stream<NCH>(w + size_t(row) * k, k, w0);
+    load_chunks_stream<NCH>(w + size_t(row1) * k, k, w1);
+    load_chunks_f32<NCH>(x, k, xv);
+    load_chunks_16<NCH>(nw, k, g);
+    rmsnorm_chunks<NCH>(xv, g, k, eps);
+    const float out0 = dot_chunks<NCH>(w0, xv), out1 = dot_chunks<NCH>(w1, xv);
+    if ((threadIdx.x & 63) == 0) {
+        y[row] = out0;
+        if (row1 != row) y[row1] = out1;
     }
 }
 
@@ -1706,28 +1723,44 @@ __global__ __launch_bounds__(256) void k_gemv_resid_dec(const float* a, const ui
 }
 
 // ---------------------------------------------------------------- 24 gemv_swiglu_dec: a[j] = silu(g_j . h) * (u_j . h)
-// R gate/up pairs per wave, as 20 gemv_norm_dec.
-template <int NCH, int R>
+template <int NCH>
 __global__ __launch_bounds__(256) void k_gemv_swiglu_dec(const float* x, const uint16_t* nw, const uint16_t* w,
                                                          float* y, int inter, int hidden, float eps) {
-    const int j = (blockIdx.x * 4 + (threadIdx.x >> 6)) * R;
+    const int j = blockIdx.x * 4 + (threadIdx.x >> 6);
     if (j >= inter) return;
-    uint4 wg[R][NCH], wu[R][NCH], g[NCH];
+    uint4 wg[NCH], wu[NCH], g[NCH];
     float xv[NCH][8];
-#pragma unroll
-    for (int r = 0; r < R; ++r) {
-        const size_t jr = size_t(min(j + r, inter - 1));
-        load_chunks_stream<NCH>(w + jr * hidden, hidden, wg[r]);
-        load_chunks_stream<NCH>(w + (size_t(inter) + jr) * hidden, hidden, wu[r]);
-    }
+    load_chunks_16<NCH>(w + size_t(j) * hidden, hidden, wg);
+    load_chunks_16<NCH>(w + size_t(inter + j) * hidden, hidden, wu);
     load_chunks_f32<NCH>(x, hidden, xv);
     load_chunks_16<NCH>(nw, hidden, g);
     rmsnorm_chunks<NCH>(xv, g, hidden, eps);
-#pragma unroll
-    for (int r = 0; r < R; ++r) {
-        const float gv = dot_chunks<NCH>(wg[r], xv);
-        const float uv = dot_chunks<NCH>(wu[r], xv);
-        if ((threadIdx.x & 63) == 0 && j + r < inter) y[j + r] = gv / (1.0f + __expf(-gv)) * uv;
+    const float gv = dot_chunks<NCH>(wg, xv);
+    const float uv = dot_chunks<NCH>(wu, xv);
+    if ((threadIdx.x & 63) == 0) y[j] = gv / (1.0f + __expf(-gv)) * uv;
+}
+
+// Two gate/up pairs per wave, as k_gemv_norm_dec2.
+template <int NCH>
+__global__ __launch_bounds__(256) void k_gemv_swiglu_dec2(const float* x, const uint16_t* nw, const uint16_t* w,
+                                                          float* y, int inter, int hidden, float eps) {
+    const int j = (blockIdx.x * 4 + (threadIdx.x >> 6)) * 2;
+    if (j >= inter) return;
+    const int j1 = min(j + 1, inter - 1);
+    uint4 wg0[NCH], wu0[NCH], wg1[NCH], wu1[NCH], g[NCH];
+    float xv[NCH][8];
+    load_chunks_stream<NCH>(w + size_t(j) * hidden, hidden, wg0);
+    load_chunks_stream<NCH>(w + size_t(inter + j) * hidden, hidden, wu0);
+    load_chunks_stream<NCH>(w + size_t(j1) * hidden, hidden, wg1);
+    load_chunks_stream<NCH>(w + size_t(inter + j1) * hidden, hidden, wu1);
+    load_chunks_f32<NCH>(x, hidden, xv);
+    load_chunks_16<NCH>(nw, hidden, g);
+    rmsnorm_chunks<NCH>(xv, g, hidden, eps);
+    const float gv0 = dot_chunks<NCH>(wg0, xv), uv0 = dot_chunks<NCH>(wu0, xv);
+    const float gv1 = dot_chunks<NCH>(wg1, xv), uv1 = dot_chunks<NCH>(wu1, xv);
+    if ((threadIdx.x & 63) == 0) {
+        y[j] = gv0 / (1.0f + __expf(-gv0)) * uv0;
+        if (j1 != j) y[j1] = gv1 / (1.0f + __expf(-gv1)) * uv1;
     }
 }
 
@@ -2333,14 +2366,14 @@ static void l_gemm_f32(const PreparedDispatch& pd, void* const* p, hipStream_t s
         hipLaunchKernelGGL((k_gemm<EPI_F32, 128, false>), grid, dim3(256), 0, s, a);
 }
 
-// Rows (or gate/up pairs) per wave of the two normed GEMVs: two where that still gives each CU two blocks of four
-// waves, for a vector of at most 2048 (the register room). One wave of a CU's SIMD with twice the loads in flight
-// streams as well as two, and half as many waves load and norm the vector. Measured with the non-temporal weight loads,
-// in a step that streams 800 MB: 12.9 -> 11.8 us for 2 x 6144 rows of 2048 (50 MB), 6.3 -> 5.8 for 4096 rows of 2048;
-// four rows 12.7 and 5.6. The residual GEMVs (2048 rows) gain nothing from either: 7.2 / 4.3 us as they are,
-// 7.2 / 4.5 with both. A whole step at that layer: 6 layers 261 -> 238 us, 4 layers 181 -> 169; with 2 layers, whose 200 MB
-// of weights the last-level cache would have kept, 95 -> 97.
-static int gemv_rows(uint32_t rows, uint32_t k) { return rows >= 4096 && k <= 2048 ? 2 : 1; }
+// Rows (or gate/up pairs) per wave of the two normed GEMVs: two where that still gives each CU two blocks of four waves,
+// for vectors of 1025 to 2048 (longer ones lack the registers, up to 1024 a wave's bytes are half). One wave of a SIMD with
+// twice the loads in flight streams as well as two, and half as many waves load and norm the vector. Measured with the
+// non-temporal weight loads, in a step that streams 800 MB: 12.9 -> 11.8 us for 2 x 6144 rows of 2048 (50 MB), 6.3 -> 5.8
+// for 4096 rows of 2048; four rows 12.7 and 5.6. The residual GEMVs (2048 rows) gain nothing from either: 7.2 / 4.3 us as
+// they are, 7.2 / 4.5 with both. A whole step at that layer: 6 layers 261 -> 238 us, 4 layers 181 -> 169; with 2 layers,
+// whose 200 MB of weights the last-level cache would have kept, 95 -> 98.
+static int gemv_rows(uint32_t rows, uint32_t k) { return rows >= 4096 && k > 1024 && k <= 2048 ? 2 : 1; }
 static uint32_t gemv_norm_blocks(uint32_t rows, uint32_t k) {
     const uint32_t per = 4u * uint32_t(gemv_rows(rows, k));
     return (rows + per - 1) / per;
@@ -2371,12 +2404,18 @@ static int nch_bucket(uint32_t k) {
 // 20 gemv_norm_dec: x, norm, w, y, n, k, eps
 static void l_gemv_norm(const PreparedDispatch& pd, void* const* p, hipStream_t s) {
     const uint32_t* w = pd.words.data();
-    const bool two = gemv_rows(w[5], w[6]) == 2;
-#define L_NORM(N)                                                                                                    \
-    hipLaunchKernelGGL((two && N <= 4 ? k_gemv_norm_dec<N, (N <= 4 ? 2 : 1)> : k_gemv_norm_dec<N, 1>),               \
-                       dim3(gemv_norm_blocks(w[5], w[6])), dim3(256), 0, s, (const float*)p[0],                      \
+#define L_NORM(KERNEL)                                                                                              \
+    hipLaunchKernelGGL(KERNEL, dim3(gemv_norm_blocks(w[5], w[6])), dim3(256), 0, s, (const float*)p[0],              \
                        (const uint16_t*)p[1], (const uint16_t*)p[2], (float*)p[3], int(w[5]), int(w[6]), f32_of(w[7]))
-    NCH_DISPATCH(w[6], L_NORM)
+#define L_NORM_1(N) L_NORM(k_gemv_norm_dec<N>)
+    if (gemv_rows(w[5], w[6]) == 1) {
+        NCH_DISPATCH(w[6], L_NORM_1)
+    } else if (nch_bucket(w[6]) == 3) {
+        L_NORM(k_gemv_norm_dec2<3>);
+    } else {
+        L_NORM(k_gemv_norm_dec2<4>);
+    }
+#undef L_NORM_1
 #undef L_NORM
 }
 
@@ -2464,12 +2503,18 @@ static void l_gemv_resid(const PreparedDispatch& pd, void* const* p, hipStream_t
 // 24 gemv_swiglu_dec: x, norm, w, y, inter, hidden, eps
 static void l_gemv_swiglu(const PreparedDispatch& pd, void* const* p, hipStream_t s) {
     const uint32_t* w = pd.words.data();
-    const bool two = gemv_rows(w[5], w[6]) == 2;
-#define L_SWIGLU(N)                                                                                                  \
-    hipLaunchKernelGGL((two && N <= 4 ? k_gemv_swiglu_dec<N, (N <= 4 ? 2 : 1)> : k_gemv_swiglu_dec<N, 1>),           \
-                       dim3(gemv_norm_blocks(w[5], w[6])), dim3(256), 0, s, (const float*)p[0],                      \
+#define L_SWIGLU(KERNEL)                                                                                              \
+    hipLaunchKernelGGL(KERNEL, dim3(gemv_norm_blocks(w[5], w[6])), dim3(256), 0, s, (const float*)p[0],              \
                        (const uint16_t*)p[1], (const uint16_t*)p[2], (float*)p[3], int(w[5]), int(w[6]), f32_of(w[7]))
-    NCH_DISPATCH(w[6], L_SWIGLU)
+#define L_SWIGLU_1(N) L_SWIGLU(k_gemv_swiglu_dec<N>)
+    if (gemv_rows(w[5], w[6]) == 1) {
+        NCH_DISPATCH(w[6], L_SWIGLU_1)
+    } else if (nch_bucket(w[6]) == 3) {
+        L_SWIGLU(k_gemv_swiglu_dec2<3>);
+    } else {
+        L_SWIGLU(k_gemv_swiglu_dec2<4>);
+    }
+#undef L_SWIGLU_1
 #undef L_SWIGLU
 }
 
