@@ -238,7 +238,22 @@ static void launch_mfma(bool vec, const float* x, const MatmulGroup& g, uint32_t
         hipLaunchKernelGGL((k_matmul_mfma<WR, WC, TM, TN, KS, D, NB, false, false>), grid, block, 0, s, x, g, m, k);
 }
 
+// k = 0: every output is an empty chain, +0. The tile kernels read element 0 of every row, which does not exist then.
+__global__ __launch_bounds__(256) void k_zero_rows(MatmulGroup group, uint32_t m) {
+    for (uint32_t i = 0; i < group.count; ++i) {
+        const uint64_t n = uint64_t(m) * group.n[i], step = uint64_t(gridDim.x) * 256u;
+        for (uint64_t e = uint64_t(blockIdx.x) * 256u + threadIdx.x; e < n; e += step) group.y[i][e] = 0.f;
+    }
+}
+
 void matmul_bf16w(const float* x, const MatmulGroup& g, uint32_t m, uint32_t k, hipStream_t s) {
+    if (k == 0) {
+        uint64_t most = 0;
+        for (uint32_t i = 0; i < g.count; ++i) most = most > g.n[i] ? most : g.n[i];
+        const uint64_t blocks = (most * m + 255) / 256;
+        hipLaunchKernelGGL(k_zero_rows, dim3(uint32_t(blocks < 4096 ? blocks : 4096)), dim3(256), 0, s, g, m);
+        return;
+    }
     bool vec = k % 8 == 0 && aligned16(x);
     uint64_t n = 0, big = 0, small = 0;
     for (uint32_t i = 0; i < g.count; ++i) {
