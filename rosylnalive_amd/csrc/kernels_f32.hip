@@ -415,10 +415,13 @@ __global__ __launch_bounds__(W == 1 ? 256 : 64 * W) void k_attention_mfma(
 #pragma unroll
         for (int st = 0; st < 16; ++st) sum = __builtin_amdgcn_mfma_f32_16x16x4f32(1.f, pf[st >> 2][st & 3], sum, 0, 0, 0);
         bs = sum[0];
-        // A key past a column's own has weight 0, which leaves the chain as it is only while its value is finite: where
-        // a block with such keys holds an infinity or a NaN, each column runs alone with those values zeroed.
+        // A key past a column's own has weight 0, and its product is a zero of its value's sign: it leaves the chain as it is
+        // while the value is finite and the chain is not -0 (a chain of products that underflow). Where a block with such
+        // keys holds an infinity or a NaN, or ends at a zero, each column runs alone with those values at -0 (a product of
+        // -0 changes no chain). The look at the ends costs 512 rows of 16 heads 52.0 -> 54.1 us, 4096 rows 1310 -> 1321.
+        const bool partial = b * 64u + 64u > first_keys;
         bool odd = false;
-        if (b * 64u + 64u > first_keys) {
+        if (partial) {
             float bad = 0.f;  // NaN once a value is not finite
 #pragma unroll
             for (int st = 0; st < 16; ++st)
@@ -441,7 +444,19 @@ __global__ __launch_bounds__(W == 1 ? 256 : 64 * W) void k_attention_mfma(
                     for (int e = 0; e < E; ++e)
                         acc[c][e] =
                             __builtin_amdgcn_mfma_f32_16x16x4f32(vr[st][c][e], pf[st >> 2][st & 3], acc[c][e], 0, 0, 0);
-            return;
+            if (!partial) return;
+            uint32_t least = ~0u;
+#pragma unroll
+            for (int c = 0; c < NC; ++c)
+#pragma unroll
+                for (int e = 0; e < E; ++e)
+#pragma unroll
+                    for (int r = 0; r < 4; ++r) {
+                        const uint32_t magnitude = __float_as_uint(acc[c][e][r]) << 1;
+                        least = magnitude < least ? magnitude : least;
+                    }
+            // (a column without keys in this block has no weights, and its state stays)
+            if (__ballot(least == 0u && b * 64u < keys) == 0) return;
         }
 #pragma unroll 1
         for (uint32_t only = 0; only < 16u; ++only) {
@@ -456,7 +471,7 @@ __global__ __launch_bounds__(W == 1 ? 256 : 64 * W) void k_attention_mfma(
                 for (int st = 0; st < 16; ++st)
 #pragma unroll
                     for (int e = 0; e < E; ++e)
-                        a[e] = __builtin_amdgcn_mfma_f32_16x16x4f32(4 * st < own ? vr[st][c][e] : 0.f,
+                        a[e] = __builtin_amdgcn_mfma_f32_16x16x4f32(4 * st < own ? vr[st][c][e] : -0.f,
                                                                     pf[st >> 2][st & 3], a[e], 0, 0, 0);
 #pragma unroll
                 for (int e = 0; e < E; ++e)
