@@ -38,7 +38,7 @@ int lrm_abi_version(void);
  * exact rules the device enforces. */
 
 /* Kernels.all / catalog.json (src/Lrm.Gpu.Core/Kernels.g.fs:27-285): ids 0..13 are the reference catalog, 14..40
- * this backend's appended fast-path kernels, 41..44 appended fp32 kernels that do several of ids 0..13 in one launch.
+ * this backend's appended fast-path kernels, 41..46 appended fp32 kernels that do several of ids 0..13 in one launch.
  * kind: 1 token, 2 u32, 3 i32, 4 f32; access: 1 read, 2 write, 3 readwrite, 4 meta; dtype_mask: bit (1 << DType code). */
 int lrm_catalog_count(void);
 int lrm_catalog_find(const char *name); /* id, or -1 */
@@ -107,13 +107,13 @@ int lrm_hip_upload(lrm_hip_device *d, int slot, uint64_t offset, const void *src
 int lrm_hip_download(lrm_hip_device *d, int slot, uint64_t offset, void *dst, uint64_t bytes);
 
 /* IGpuBackend.LoadKernels / IKernelSet (Backend.fs:104-108,144-147): the gfx950 code objects are part of this
- * library. Loads the reference kernel set (catalog ids 0-13, Kernels.g.fs:27-285, and ids 41-44, which give the same
+ * library. Loads the reference kernel set (catalog ids 0-13, Kernels.g.fs:27-285, and ids 41-46, which give the same
  * bits as the sequences of those that they stand for), which keeps the BatchInvariance contract
  * (docs/contracts/batch-invariance.md:7-12). The shader-set hash, which fills ExecutionClass.ShaderSetHash
  * (ExecutionClass.fs:58), is the SHA-256 of the set's name and the library file's SHA-256. Runs the fp32 denormal
  * probe (Backend.fs:457-547): mode 1 preserve, 2 flush, 3 mixed. */
 int lrm_hip_load_kernels(lrm_hip_device *d, uint8_t shader_set_hash[32]);
-/* An extension of LoadKernels: the set to load, once per backend. LRM_HIP_KERNELS_FAST is every id (0-44, the
+/* An extension of LoadKernels: the set to load, once per backend. LRM_HIP_KERNELS_FAST is every id (0-46, the
  * appended fast path included) under its own shader-set hash, so its results form their own ExecutionClass: it only
  * claims that the same work on the same inputs gives the same bits (the row count chooses its k-split and attention
  * splits; its prefill and decode kernels sum in different orders), and no bit-identity claim crosses the two sets. */

@@ -448,8 +448,25 @@ static std::vector<KernelSpec> base_catalog() {
 }
 
 // The appended entries of this backend: the fast path (ids 14..40), defined next to its kernels' host code, then fusions
-// of the reference's own kernels (ids 41..44), whose results equal the dispatches they stand for bit for bit.
+// of the reference's own kernels (ids 41..46), whose results equal the dispatches they stand for bit for bit.
 std::vector<KernelSpec> fast_catalog();
+
+// The checks of 43 and 45. w: rows, q_heads, kv_heads, head_dim, pos0; norms: q_norm's field, with k_norm and the tables after
+// it; caches: k_cache's, with v_cache after it.
+static void need_heads(const char* n, const uint32_t* w, const uint32_t* c, int norms, int caches) {
+    const int64_t rows = w[0], qh = w[1], kvh = w[2], hd = w[3], pos0 = w[4];
+    if (qh < 1 || kvh < 1) contract_fail("%s: heads must be at least 1", n);
+    if (hd < 2 || hd % 2 || hd > 8192) contract_fail("%s: head_dim must be even, 2 to 8192", n);
+    need(c, 0, rows * qh * hd, n, "q");
+    need(c, 1, rows * kvh * hd, n, "k");
+    need(c, 2, rows * kvh * hd, n, "v");
+    need(c, norms, hd, n, "q_norm");
+    need(c, norms + 1, hd, n, "k_norm");
+    need(c, norms + 2, (pos0 + rows) * (hd / 2), n, "cos_table");
+    need(c, norms + 3, (pos0 + rows) * (hd / 2), n, "sin_table");
+    need(c, caches, (pos0 + rows) * kvh * hd, n, "k_cache");
+    need(c, caches + 1, (pos0 + rows) * kvh * hd, n, "v_cache");
+}
 
 static std::vector<KernelSpec> fused_catalog() {
     std::vector<KernelSpec> c;
@@ -483,7 +500,7 @@ static std::vector<KernelSpec> fused_catalog() {
                      }
                  }});
     // 43 qk_norm_rope_append: rmsnorm_rows and rope_apply on q's and k's heads, copy_rows of k and v into the caches' rows
-    // pos0 ..
+    // pos0 ..; 45 qk_norm_rope_append_all also writes the normed heads (qn, kn) and the rotated k rows (kr)
     c.push_back({"qk_norm_rope_append", "attention", {256, 1, 1}, false,
                  [](const uint32_t* w) { return Grid3{w[11], int64_t(w[12]) + 2 * int64_t(w[13]), 1}; },
                  {TOK_R("q", DT(F32)), TOK_R("k", DT(F32)), TOK_R("v", DT(F32)), TOK_R("q_norm", DT(BF16)),
@@ -491,20 +508,8 @@ static std::vector<KernelSpec> fused_catalog() {
                   TOK_W("qr", DT(F32), nullptr), TOK_W("k_cache", DT(F32), nullptr), TOK_W("v_cache", DT(F32), nullptr),
                   U32F("rows"), U32F("q_heads"), U32F("kv_heads"), U32F("head_dim"), U32F("pos0"), F32F("eps")},
                  [](const uint32_t* w, const uint32_t* c) {
-                     const char* n = "qk_norm_rope_append";
-                     const int64_t rows = w[11], qh = w[12], kvh = w[13], hd = w[14], pos0 = w[15];
-                     if (qh < 1 || kvh < 1) contract_fail("%s: heads must be at least 1", n);
-                     if (hd < 2 || hd % 2 || hd > 8192) contract_fail("%s: head_dim must be even, 2 to 8192", n);
-                     need(c, 0, rows * qh * hd, n, "q");
-                     need(c, 1, rows * kvh * hd, n, "k");
-                     need(c, 2, rows * kvh * hd, n, "v");
-                     need(c, 3, hd, n, "q_norm");
-                     need(c, 4, hd, n, "k_norm");
-                     need(c, 5, (pos0 + rows) * (hd / 2), n, "cos_table");
-                     need(c, 6, (pos0 + rows) * (hd / 2), n, "sin_table");
-                     need(c, 7, rows * qh * hd, n, "qr");
-                     need(c, 8, (pos0 + rows) * kvh * hd, n, "k_cache");
-                     need(c, 9, (pos0 + rows) * kvh * hd, n, "v_cache");
+                     need_heads("qk_norm_rope_append", w + 11, c, 3, 8);
+                     need(c, 7, int64_t(w[11]) * w[12] * w[14], "qk_norm_rope_append", "qr");
                  }});
     // 44 add_rmsnorm_rows: r = a + b (add), y = rmsnorm_rows(r, w)
     c.push_back({"add_rmsnorm_rows", "basic", {256, 1, 1}, true, [](const uint32_t* w) { return Grid3{w[6], 1, 1}; },
@@ -518,6 +523,40 @@ static std::vector<KernelSpec> fused_catalog() {
                      need(c, 2, w[7], "add_rmsnorm_rows", "w");
                      need(c, 3, n, "add_rmsnorm_rows", "r");
                      need(c, 4, n, "add_rmsnorm_rows", "y");
+                 }});
+    // 45 qk_norm_rope_append_all
+    c.push_back({"qk_norm_rope_append_all", "attention", {256, 1, 1}, false,
+                 [](const uint32_t* w) { return Grid3{w[14], int64_t(w[15]) + 2 * int64_t(w[16]), 1}; },
+                 {TOK_R("q", DT(F32)), TOK_R("k", DT(F32)), TOK_R("v", DT(F32)), TOK_R("q_norm", DT(BF16)),
+                  TOK_R("k_norm", DT(BF16)), TOK_R("cos_table", DT(F32)), TOK_R("sin_table", DT(F32)),
+                  TOK_W("qn", DT(F32), nullptr), TOK_W("qr", DT(F32), nullptr), TOK_W("kn", DT(F32), nullptr),
+                  TOK_W("kr", DT(F32), nullptr), TOK_W("k_cache", DT(F32), nullptr), TOK_W("v_cache", DT(F32), nullptr),
+                  U32F("rows"), U32F("q_heads"), U32F("kv_heads"), U32F("head_dim"), U32F("pos0"), F32F("eps")},
+                 [](const uint32_t* w, const uint32_t* c) {
+                     const char* n = "qk_norm_rope_append_all";
+                     need_heads(n, w + 14, c, 3, 11);
+                     const int64_t q = int64_t(w[14]) * w[15] * w[17], k = int64_t(w[14]) * w[16] * w[17];
+                     need(c, 7, q, n, "qn");
+                     need(c, 8, q, n, "qr");
+                     need(c, 9, k, n, "kn");
+                     need(c, 10, k, n, "kr");
+                 }});
+    // 46 add_rmsnorm_rows_tail: add_rmsnorm_rows, and the last `tail` rows of y again as y_tail (copy_rows)
+    c.push_back({"add_rmsnorm_rows_tail", "basic", {256, 1, 1}, true, [](const uint32_t* w) { return Grid3{w[7], 1, 1}; },
+                 {TOK_R("a", DT(F32)), TOK_R("b", DT(F32)), TOK_R("w", DT(BF16)), TOK_W("r", DT(F32), nullptr),
+                  TOK_W("y", DT(F32), nullptr), TOK_W("y_tail", DT(F32), nullptr), U32F("rows"), U32F("cols"), F32F("eps"),
+                  U32F("tail")},
+                 [](const uint32_t* w, const uint32_t* c) {
+                     const char* n = "add_rmsnorm_rows_tail";
+                     if (w[8] < 1) contract_fail("%s: cols must be at least 1", n);
+                     if (w[10] < 1 || w[10] > w[7]) contract_fail("%s: tail must be 1 to rows", n);
+                     const int64_t e = int64_t(w[7]) * w[8];
+                     need(c, 0, e, n, "a");
+                     need(c, 1, e, n, "b");
+                     need(c, 2, w[8], n, "w");
+                     need(c, 3, e, n, "r");
+                     need(c, 4, e, n, "y");
+                     need(c, 5, int64_t(w[10]) * w[8], n, "y_tail");
                  }});
     return c;
 }

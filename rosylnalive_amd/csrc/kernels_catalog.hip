@@ -1,7 +1,7 @@
 // The reference catalog's kernels 0..13 (docs/contracts/kernel-abi.md "The catalog at contracts-v1") for gfx950:
 // fp32 activations, bf16 weights, the arithmetic of CpuRef F32 where the catalog asks for it. These are the parity
 // path of the device (the executor's fp32 mode), with its contractions in kernels_f32.hip and, at the end of the catalog
-// (ids 41..44), fusions of it with the same bits; the bf16 performance kernels are in kernels_fast.hip.
+// (ids 41..46), fusions of it with the same bits; the bf16 performance kernels are in kernels_fast.hip.
 //
 // Built with -ffp-contract=off: every product is rounded before the following add unless fmaf is written, as CpuRef
 // does (docs/contracts/cpu-reference.md rules 2 and 4). Division and sqrtf are IEEE (hipcc's default
@@ -136,18 +136,21 @@ __global__ void k_copy_rows(const uint32_t* src, uint32_t* dst, uint32_t rows, u
     dst[(uint64_t(dr0) + r) * ds + c] = src[(uint64_t(sr0) + r) * ss + c];
 }
 
-// ================================================================ fusions (ids 41..44)
+// ================================================================ fusions (ids 41..46)
 // The float32 forward's runs of small dispatches as one launch each (a launch costs 2-5 us, most of these kernels' time),
 // with the arithmetic of the kernels they replace, operation for operation.
 
-// ---------------------------------------------------------------- 43 qk_norm_rope_append
+// ---------------------------------------------------------------- 43 qk_norm_rope_append, 45 qk_norm_rope_append_all
 // One block per (row, head of q, k or v): rmsnorm_rows on the head, rope_apply, and the row's place: qr for q, the caches
-// for k and v (v as it is).
+// for k and v (v as it is). 45 also writes what the separate kernels leave: the normed heads and the rotated k rows.
+struct QkKept {
+    float *qn, *kn, *kr;  // null: not written
+};
 __global__ __launch_bounds__(256) void k_qk_norm_rope_append(const float* q, const float* k, const float* v,
                                                              const uint16_t* qn, const uint16_t* kn, const float* cos_t,
                                                              const float* sin_t, float* qr, float* kc, float* vc,
-                                                             uint32_t qh, uint32_t kvh, uint32_t hd, uint32_t pos0,
-                                                             float eps) {
+                                                             QkKept kept, uint32_t qh, uint32_t kvh, uint32_t hd,
+                                                             uint32_t pos0, float eps) {
     __shared__ float red[4];
     extern __shared__ float xn[];  // the normed head
     const uint32_t r = blockIdx.x, h = blockIdx.y, half = hd / 2u;
@@ -160,7 +163,10 @@ __global__ __launch_bounds__(256) void k_qk_norm_rope_append(const float* q, con
     const bool is_q = h < qh;
     const float* xr = is_q ? q + (size_t(r) * qh + h) * hd : k + (size_t(r) * kvh + (h - qh)) * hd;
     const uint16_t* w = is_q ? qn : kn;
-    float* yr = is_q ? qr + (size_t(r) * qh + h) * hd : kc + (pos * kvh + (h - qh)) * hd;
+    const size_t row = is_q ? (size_t(r) * qh + h) * hd : (size_t(r) * kvh + (h - qh)) * hd;  // of the kept tensors
+    float* yr = is_q ? qr + row : kc + (pos * kvh + (h - qh)) * hd;
+    float* normed = is_q ? kept.qn : kept.kn;
+    float* rotated = is_q ? nullptr : kept.kr;
     float ss = 0.f;
     for (uint32_t c = threadIdx.x; c < hd; c += 256u) ss = fmaf(xr[c], xr[c], ss);
     ss = block_sum_256(ss, red);
@@ -169,6 +175,7 @@ __global__ __launch_bounds__(256) void k_qk_norm_rope_append(const float* q, con
     for (uint32_t c = threadIdx.x; c < hd; c += 256u) {
         const float xv = xr[c] * rr;
         xn[c] = widen(w[c]) * xv;
+        if (normed) normed[row + c] = xn[c];
     }
     __syncthreads();
     for (uint32_t i = threadIdx.x; i < half; i += 256u) {
@@ -177,16 +184,23 @@ __global__ __launch_bounds__(256) void k_qk_norm_rope_append(const float* q, con
         const float ac = a * c, bs = b * s, bc = b * c, as = a * s;
         yr[i] = ac - bs;
         yr[i + half] = bc + as;
+        if (rotated) {
+            rotated[row + i] = ac - bs;
+            rotated[row + i + half] = bc + as;
+        }
     }
 }
 
-// ---------------------------------------------------------------- 44 add_rmsnorm_rows: r = a + b, y = rmsnorm_rows(r)
+// ---------------------------------------------------------------- 44 add_rmsnorm_rows, 46 add_rmsnorm_rows_tail
+// r = a + b, y = rmsnorm_rows(r); 46 also writes y's last `tail` rows to y_tail.
 __global__ __launch_bounds__(256) void k_add_rmsnorm_rows(const float* a, const float* b, const uint16_t* w, float* r,
-                                                          float* y, uint32_t rows, uint32_t cols, float eps) {
+                                                          float* y, float* y_tail, uint32_t rows, uint32_t cols, float eps,
+                                                          uint32_t tail) {
     __shared__ float red[4];
     const uint32_t row = linear_group();
     if (row >= rows) return;
     const size_t at = size_t(row) * cols;
+    float* yt = row + tail >= rows && tail ? y_tail + size_t(row + tail - rows) * cols : nullptr;
     constexpr int KEEP = 8;  // of the row's sums per thread (2048 columns); the rest are read back
     float x[KEEP];
     float ss = 0.f;
@@ -211,13 +225,15 @@ __global__ __launch_bounds__(256) void k_add_rmsnorm_rows(const float* a, const 
     for (int i = 0; i < KEEP; ++i) {
         const uint32_t c = threadIdx.x + 256u * i;
         if (c < cols) {
-            const float xv = x[i] * rr;
-            y[at + c] = widen(w[c]) * xv;
+            const float xv = x[i] * rr, v = widen(w[c]) * xv;
+            y[at + c] = v;
+            if (yt) yt[c] = v;
         }
     }
     for (uint32_t c = threadIdx.x + 256u * KEEP; c < cols; c += 256u) {
-        const float xv = r[at + c] * rr;
-        y[at + c] = widen(w[c]) * xv;
+        const float xv = r[at + c] * rr, v = widen(w[c]) * xv;
+        y[at + c] = v;
+        if (yt) yt[c] = v;
     }
 }
 
@@ -429,18 +445,34 @@ static void l_qk_norm_rope_append(const PreparedDispatch& pd, void* const* p, hi
     const uint32_t* w = pd.words.data();
     hipLaunchKernelGGL(k_qk_norm_rope_append, dim3(w[11], w[12] + 2 * w[13]), dim3(256), w[14] * 4, s, (const float*)p[0],
                        (const float*)p[1], (const float*)p[2], (const uint16_t*)p[3], (const uint16_t*)p[4],
-                       (const float*)p[5], (const float*)p[6], (float*)p[7], (float*)p[8], (float*)p[9], w[12], w[13],
-                       w[14], w[15], f32_of(w[16]));
+                       (const float*)p[5], (const float*)p[6], (float*)p[7], (float*)p[8], (float*)p[9], QkKept{}, w[12],
+                       w[13], w[14], w[15], f32_of(w[16]));
+}
+// 45 qk_norm_rope_append_all: q, k, v, q_norm, k_norm, cos, sin, qn, qr, kn, kr, k_cache, v_cache, rows, q_heads, kv_heads,
+// head_dim, pos0, eps
+static void l_qk_norm_rope_append_all(const PreparedDispatch& pd, void* const* p, hipStream_t s) {
+    const uint32_t* w = pd.words.data();
+    hipLaunchKernelGGL(k_qk_norm_rope_append, dim3(w[14], w[15] + 2 * w[16]), dim3(256), w[17] * 4, s, (const float*)p[0],
+                       (const float*)p[1], (const float*)p[2], (const uint16_t*)p[3], (const uint16_t*)p[4],
+                       (const float*)p[5], (const float*)p[6], (float*)p[8], (float*)p[11], (float*)p[12],
+                       QkKept{(float*)p[7], (float*)p[9], (float*)p[10]}, w[15], w[16], w[17], w[18], f32_of(w[19]));
 }
 // 44 add_rmsnorm_rows: a, b, w, r, y, rows, cols, eps
 static void l_add_rmsnorm(const PreparedDispatch& pd, void* const* p, hipStream_t s) {
     const uint32_t* w = pd.words.data();
     hipLaunchKernelGGL(k_add_rmsnorm_rows, phys(pd), dim3(256), 0, s, (const float*)p[0], (const float*)p[1],
-                       (const uint16_t*)p[2], (float*)p[3], (float*)p[4], w[6], w[7], f32_of(w[8]));
+                       (const uint16_t*)p[2], (float*)p[3], (float*)p[4], (float*)nullptr, w[6], w[7], f32_of(w[8]), 0u);
+}
+// 46 add_rmsnorm_rows_tail: a, b, w, r, y, y_tail, rows, cols, eps, tail
+static void l_add_rmsnorm_tail(const PreparedDispatch& pd, void* const* p, hipStream_t s) {
+    const uint32_t* w = pd.words.data();
+    hipLaunchKernelGGL(k_add_rmsnorm_rows, phys(pd), dim3(256), 0, s, (const float*)p[0], (const float*)p[1],
+                       (const uint16_t*)p[2], (float*)p[3], (float*)p[4], (float*)p[5], w[7], w[8], f32_of(w[9]), w[10]);
 }
 
 const LaunchFn* fused_launchers() {
-    static const LaunchFn t[4] = {l_matmul_triple, l_matmul_pair, l_qk_norm_rope_append, l_add_rmsnorm};
+    static const LaunchFn t[6] = {l_matmul_triple, l_matmul_pair,           l_qk_norm_rope_append,
+                                  l_add_rmsnorm,   l_qk_norm_rope_append_all, l_add_rmsnorm_tail};
     return t;
 }
 

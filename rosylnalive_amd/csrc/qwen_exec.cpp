@@ -647,7 +647,7 @@ uint32_t QwenExec::forward_fp32(int pos0, int T, float* logits, int lr) {
     const uint32_t LR = uint32_t(c.taps ? T : lr);
     if (LR > dev_.table().row(tk("logits")).count() / V) arg_fail("%u logits rows exceed the logits tensor", LR);
     CommandList* l = dev_.begin();
-    if (!c.taps) {  // the same operations in fewer launches: nobody reads what the separate ones leave between
+    if (!c.taps) {  // the same operations in fewer launches; what the separate ones leave behind, the last layer writes too
         dispatch(l, "embed_gather_bf16", {tk("ids"), tk("model.embed_tokens.weight"), tk("x"), U, H, V});
         dispatch(l, "rmsnorm_rows", {tk("x"), tk(lname(0, kLayerWeights[0])), tk("h"), U, H, eps});
         for (int i = 0; i < c.layers; ++i) {
@@ -655,9 +655,16 @@ uint32_t QwenExec::forward_fp32(int pos0, int T, float* logits, int lr) {
             auto w = [&](int k) { return tk(lname(i, kLayerWeights[k])); };
             const bool last = i + 1 == c.layers;
             dispatch(l, "matmul_bf16w_triple", {tk("h"), w(1), w(2), w(3), tk("q"), tk("k"), tk("v"), U, QC, KC, KC, H});
-            dispatch(l, "qk_norm_rope_append",
-                     {tk("q"), tk("k"), tk("v"), w(5), w(6), tk("rope.cos"), tk("rope.sin"), tk("qr"), tk(p + "k_cache"),
-                      tk(p + "v_cache"), U, uint32_t(c.heads), uint32_t(c.kv_heads), HD, uint32_t(pos0), eps});
+            if (!last)
+                dispatch(l, "qk_norm_rope_append",
+                         {tk("q"), tk("k"), tk("v"), w(5), w(6), tk("rope.cos"), tk("rope.sin"), tk("qr"),
+                          tk(p + "k_cache"), tk(p + "v_cache"), U, uint32_t(c.heads), uint32_t(c.kv_heads), HD,
+                          uint32_t(pos0), eps});
+            else
+                dispatch(l, "qk_norm_rope_append_all",
+                         {tk("q"), tk("k"), tk("v"), w(5), w(6), tk("rope.cos"), tk("rope.sin"), tk("qn"), tk("qr"),
+                          tk("kn"), tk("kr"), tk(p + "k_cache"), tk(p + "v_cache"), U, uint32_t(c.heads),
+                          uint32_t(c.kv_heads), HD, uint32_t(pos0), eps});
             dispatch(l, "attention_gqa_causal", {tk("qr"), tk(p + "k_cache"), tk(p + "v_cache"), tk("o"), U, 0,
                                                  uint32_t(pos0), uint32_t(c.heads), uint32_t(c.kv_heads), HD, scale});
             dispatch(l, "matmul_bf16w", {tk("o"), w(4), tk("oo"), U, H, QC});
@@ -665,13 +672,15 @@ uint32_t QwenExec::forward_fp32(int pos0, int T, float* logits, int lr) {
             dispatch(l, "matmul_bf16w_pair", {tk("h2"), w(8), w(9), tk("g"), tk("u"), U, I, I, H});
             dispatch(l, "silu_mul", {tk("g"), tk("u"), tk("d"), U * I});
             dispatch(l, "matmul_bf16w", {tk("d"), w(10), tk("dd"), U, H, I});
-            dispatch(l, "add_rmsnorm_rows",
-                     {tk("r"), tk("dd"), last ? tk("model.norm.weight") : tk(lname(i + 1, kLayerWeights[0])), tk("x"),
-                      tk(last ? "f" : "h"), U, H, eps});
+            if (!last)
+                dispatch(l, "add_rmsnorm_rows",
+                         {tk("r"), tk("dd"), tk(lname(i + 1, kLayerWeights[0])), tk("x"), tk("h"), U, H, eps});
+            else
+                dispatch(l, "add_rmsnorm_rows_tail",
+                         {tk("r"), tk("dd"), tk("model.norm.weight"), tk("x"), tk("f"), tk("f_last"), U, H, eps, LR});
             flush(l);
         }
-        if (LR < U) dispatch(l, "copy_rows", {tk("f"), tk("f_last"), LR, H, U - LR, 0, H, H});
-        dispatch(l, "matmul_bf16w", {tk(LR < U ? "f_last" : "f"), tk("model.embed_tokens.weight"), tk("logits"), LR, V, H});
+        dispatch(l, "matmul_bf16w", {tk("f_last"), tk("model.embed_tokens.weight"), tk("logits"), LR, V, H});
         dispatch(l, "argmax_rows", {tk("logits"), tk("argmax"), LR, V});
         return finish_fp32(l, logits, lr, LR);
     }

@@ -5,7 +5,7 @@
 // dispatches.
 //
 // Two modes:
-//   Fp32 - the reference catalog kernels (ids 0..13; without taps their fused forms 41..44, the same bits): fp32
+//   Fp32 - the reference catalog kernels (ids 0..13; without taps their fused forms 41..46, the same bits): fp32
 //          activations and an fp32 token-major KV cache, as every reference GPU keeps. This is the parity path against CpuRef F32.
 //   Fast - the appended kernels: bf16 weights, fp16 MFMA operands in prefill (an exact on-device fp16 copy of each
 //          matrix, fp16-rounded activations), fp32 residual stream, a head-major fp16 KV cache, fused

@@ -405,7 +405,7 @@ class HipBackend:
     KERNEL_SETS = {"reference": 0, "fast": 1}
 
     def load_kernels(self, kernel_set: str = "reference") -> bytes:
-        """LoadKernels, once per backend: "reference" (catalog ids 0-13 and 41-44, the BatchInvariance contract) or "fast"
+        """LoadKernels, once per backend: "reference" (catalog ids 0-13 and 41-46, the BatchInvariance contract) or "fast"
         (every id, its own ExecutionClass: same work, same inputs, same bits, and no more). Returns the set's
         shader-set hash."""
         h = C.create_string_buffer(32)
