@@ -2239,8 +2239,13 @@ static int small_tile(uint64_t full, uint64_t rows64, uint64_t half) {
 static uint64_t tiles_of(uint64_t m, uint64_t rows, uint64_t n, uint64_t cols) {
     return ((m + rows - 1) / rows) * ((n + cols - 1) / cols);
 }
-static bool qkv_rows64(uint32_t m, uint32_t heads) {
-    return small_tile(tiles_of(m, 128, heads, 1), tiles_of(m, 64, heads, 1), 0) == 1;
+// gemm_qkv_rope's tile, one head wide: 128 rows on the direct-to-LDS loop (-1), or the register loop's 128 (0) or 64 (1)
+static int qkv_tile(uint32_t m, uint32_t heads) {
+    if (two_per_cu(dim3(heads, (m + 127) / 128))) return -1;
+    return small_tile(tiles_of(m, 128, heads, 1), tiles_of(m, 64, heads, 1), 0);
+}
+static dim3 qkv_grid(uint32_t m, uint32_t heads) {
+    return dim3(heads, qkv_tile(m, heads) == 1 ? (m + 63) / 64 : (m + 127) / 128);
 }
 
 // 15 gemm_qkv_rope: h, w, q_norm, k_norm, cos, sin, q, k_cache, v_cache, m, hidden, q_heads, kv_heads, pos0, max_pos,
@@ -2261,13 +2266,13 @@ static void l_gemm_qkv(const PreparedDispatch& pd, void* const* p, hipStream_t s
     a.pos0 = int(w[14]);
     a.max_pos = int(w[15]);
     a.eps = f32_of(w[16]);
-    const dim3 grid(uint32_t(qh + 2 * kvh), (w[10] + GBM - 1) / GBM);
-    if (two_per_cu(grid))
-        hipLaunchKernelGGL((k_gemm<EPI_QKV, 128, true>), grid, dim3(256), 0, s, a);
-    else if (qkv_rows64(w[10], qh + 2 * kvh))
-        hipLaunchKernelGGL((k_gemm<EPI_QKV, 128, false, 64>), dim3(grid.x, (w[10] + 63) / 64), dim3(256), 0, s, a);
-    else
-        hipLaunchKernelGGL((k_gemm<EPI_QKV, 128, false>), grid, dim3(256), 0, s, a);
+    const uint32_t heads = w[12] + 2 * w[13];
+    const dim3 grid = qkv_grid(w[10], heads);
+    switch (qkv_tile(w[10], heads)) {
+        case -1: hipLaunchKernelGGL((k_gemm<EPI_QKV, 128, true>), grid, dim3(256), 0, s, a); break;
+        case 0: hipLaunchKernelGGL((k_gemm<EPI_QKV, 128, false>), grid, dim3(256), 0, s, a); break;
+        default: hipLaunchKernelGGL((k_gemm<EPI_QKV, 128, false, 64>), grid, dim3(256), 0, s, a); break;
+    }
 }
 
 // 16 attention_prefill_f16: q, k_cache, v_cache, y, workspace, rows, past, q_heads, kv_heads, max_pos, scale
@@ -2777,8 +2782,8 @@ std::vector<KernelSpec> fast_catalog() {
     // 15 gemm_qkv_rope
     c.push_back({"gemm_qkv_rope", "fast", {256, 1, 1}, false,
                  [](const uint32_t* w) {
-                     const uint32_t heads = w[12] + 2 * w[13], rows = qkv_rows64(w[10], heads) ? 64 : 128;
-                     return Grid3{heads, (int64_t(w[10]) + rows - 1) / rows, 1};
+                     const dim3 g = qkv_grid(w[10], w[12] + 2 * w[13]);
+                     return Grid3{g.x, g.y, g.z};
                  },
                  {TOK_R("h", DT(F16)), TOK_R("w", DT(F16)), TOK_R("q_norm", DT(BF16)), TOK_R("k_norm", DT(BF16)),
                   TOK_R("cos_table", DT(F32)), TOK_R("sin_table", DT(F32)), TOK_W("q", DT(F16)),
