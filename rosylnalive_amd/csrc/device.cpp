@@ -466,7 +466,6 @@ uint64_t Device::submit(CommandList* l, uint32_t repeat) {
     HIPC(hipSetDevice(index_));
     Pending pend{};
     pend.dispatches = l->dispatches_ * int(repeat);
-    pend.owned = nullptr;
     if (!l->reusable_) {
         // One-shot: launch every command now, with timer events and per-dispatch timing as asked.
         std::vector<std::pair<hipEvent_t, hipEvent_t>> tev(l->timer_names_.size());
@@ -520,7 +519,6 @@ uint64_t Device::submit(CommandList* l, uint32_t repeat) {
         pend.timer_events = all;
         pend.timer_names = names;
         l->closed_ = true;
-        pend.owned = l;
     } else if (!graphs_enabled()) {
         // Profilers that cannot follow stream capture: replay by launching the recorded commands directly.
         if (!l->timer_names_.empty()) contract_fail("a reusable list cannot hold timers");

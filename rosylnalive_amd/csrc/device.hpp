@@ -239,7 +239,6 @@ class Device {
         std::vector<std::pair<hipEvent_t, hipEvent_t>> timer_events;
         std::vector<std::string> timer_names;
         int dispatches;
-        CommandList* owned;  // one-shot list to free after completion
     };
     std::map<uint64_t, Pending> pending_;
     std::map<uint64_t, Completion> done_;  // the last kKeptCompletions waited on, by fence

@@ -1,8 +1,10 @@
-"""The words a call exchanges with the device: token ids on either side of the count up to which kernels carry them."""
+"""The words a call exchanges with the device (token ids on either side of the count up to which kernels carry them), and its
+command lists released before they are waited for."""
 import numpy as np
 import pytest
 
-from rosylnalive_amd.gpu_core import HipBackend
+from gpu_session import Session
+from rosylnalive_amd.gpu_core import DType, HipBackend
 from rosylnalive_amd.qwen import QwenConfig, QwenModel, synthetic_ids, synthetic_weights
 
 pytestmark = pytest.mark.gpu
@@ -23,3 +25,27 @@ def test_ids_reach_the_device(t):
         m.close()
         b.close()
     assert got[0] == got[1]
+
+
+def test_one_shot_lists_released_before_the_wait():
+    """A submission keeps nothing of its one-shot list: lists released, and their memory used again, before the waits."""
+    n = 1 << 20
+    x = np.arange(n, dtype=np.float32)
+    t = {"x0": (DType.F32, (n,), 0, x)}
+    t.update({f"x{i}": (DType.F32, (n,), 0, None) for i in range(1, 9)})
+    s = Session(t)
+    try:
+        fences = []
+        for i in range(8):
+            cl = s.backend.begin()
+            timer = cl.begin_timer(f"part {i}")
+            cl.dispatch("scale_f32", s.fields("scale_f32", x=f"x{i}", y=f"x{i + 1}", n=n, a=2.0))
+            cl.end_timer(timer)
+            fences.append(s.backend.submit(cl))
+            cl.release()
+        for i, f in enumerate(fences):
+            c = s.backend.wait(f)
+            assert c.dispatches == 1 and [r.name for r in c.timers] == [f"part {i}"]
+        assert np.array_equal(s.read("x8"), x * 256)
+    finally:
+        s.close()
