@@ -1033,7 +1033,7 @@ void QwenExec::put_state(const int32_t* ids, const int32_t* pos, uint32_t step) 
     st[size_t(2 * B)] = step;
     dev_.put_words(ptr("dec.state"), st.data(), st.size());
     dec_state_ = std::move(st);
-    dec_ids_ = 0;
+    dec_ids_.clear();
 }
 
 void QwenExec::run_decode_steps(int steps) {
@@ -1043,7 +1043,8 @@ void QwenExec::run_decode_steps(int steps) {
     if (dec_exposed_) dec_state_.clear();
     std::vector<uint32_t> st;
     st.swap(dec_state_);  // (not known again until this run has succeeded)
-    dec_ids_ = 0;
+    std::vector<uint32_t> ids;
+    ids.swap(dec_ids_);
     if (st.empty()) {
         st.resize(size_t(2 * B + 2));
         download_tensor("dec.state", st.data(), st.size() * 4);
@@ -1055,11 +1056,11 @@ void QwenExec::run_decode_steps(int steps) {
     sync_f16();  // the batched step's skinny GEMMs read the fp16 copies: weights set since the last forward
     hip_check(hipEventRecord(ev_[0], dev_.stream()), "event");
     uint64_t f = dev_.submit(decode_list_, uint32_t(steps));
-    // the ids of this sequence of runs so far, where they fit
-    const uint64_t total = (uint64_t(st[size_t(2 * B)]) + uint64_t(steps)) * uint64_t(B);
-    const uint32_t nids = dec_exposed_ || total > Device::kHostIdWords ? 0u : uint32_t(total);
-    dev_.collect(true, nullptr, persist_ ? static_cast<const uint32_t*>(ptr("dec.exchange")) + 1 : nullptr, ptr("dec.out_ids"),
-                 nids);
+    // this run's ids, where the host words hold them: they follow the earlier runs' in dec_ids_
+    const uint64_t id0 = uint64_t(st[size_t(2 * B)]) * uint64_t(B), run = uint64_t(steps) * uint64_t(B);
+    const uint32_t nids = dec_exposed_ || run > Device::kHostIdWords ? 0u : uint32_t(run);
+    dev_.collect(true, nullptr, persist_ ? static_cast<const uint32_t*>(ptr("dec.exchange")) + 1 : nullptr,
+                 static_cast<const uint32_t*>(ptr("dec.out_ids")) + id0, nids);
     hip_check(hipEventRecord(ev_[1], dev_.stream()), "event");
     hip_check(hipEventSynchronize(ev_[1]), "event");
     dev_.wait(f);
@@ -1085,16 +1086,22 @@ void QwenExec::run_decode_steps(int steps) {
     for (int b = 0; b < B; ++b) st[size_t(b)] += uint32_t(steps);
     st[size_t(2 * B)] += uint32_t(steps);
     dec_state_ = std::move(st);
-    dec_ids_ = int(nids);
+    if (ids.empty()) dec_id0_ = id0;
+    if (dec_id0_ + ids.size() == id0 && nids) {
+        const volatile uint32_t* w = dev_.host_words() + Device::kHostIds;
+        ids.insert(ids.end(), w, w + nids);
+        dec_ids_ = std::move(ids);
+    }
 }
 
-void QwenExec::read_decode_ids(int32_t* out, int count) {
-    if (count < 0 || int64_t(count) > int64_t(cfg_.max_pos) * cfg_.batch) arg_fail("count %d", count);
-    if (count <= dec_ids_ && !dec_exposed_) {
-        for (int i = 0; i < count; ++i) out[i] = int32_t(dev_.host_words()[Device::kHostIds + uint32_t(i)]);
+void QwenExec::read_decode_ids(int32_t* out, int count, int first) {
+    if (count < 0 || int64_t(first) + count > int64_t(cfg_.max_pos) * cfg_.batch) arg_fail("count %d", count);
+    const uint64_t lo = uint64_t(first), n = uint64_t(count);
+    if (!dec_exposed_ && lo >= dec_id0_ && lo + n <= dec_id0_ + dec_ids_.size()) {
+        for (uint64_t i = 0; i < n; ++i) out[i] = int32_t(dec_ids_[lo - dec_id0_ + i]);
         return;
     }
-    download_tensor("dec.out_ids", out, uint64_t(count) * 4);
+    download_tensor("dec.out_ids", out, n * 4, lo * 4);
 }
 
 void QwenExec::greedy(const int32_t* prompt, int plen, int steps, int32_t* out) {
@@ -1112,12 +1119,9 @@ void QwenExec::greedy(const int32_t* prompt, int plen, int steps, int32_t* out) 
         set_decode_state(&i0, &pos);
         put_state(&i0, &pos, 1);
         run_decode_steps(steps - 1);
-        std::vector<int32_t> ids(static_cast<size_t>(steps));
-        read_decode_ids(ids.data(), steps);
-        for (int s = 1; s < steps; ++s) {
-            if (uint32_t(ids[size_t(s)]) == 0xFFFFFFFFu) throw std::runtime_error("greedy: argmax of a row that holds a NaN");
-            out[s] = ids[size_t(s)];
-        }
+        read_decode_ids(out + 1, steps - 1, 1);
+        for (int s = 1; s < steps; ++s)
+            if (uint32_t(out[s]) == 0xFFFFFFFFu) throw std::runtime_error("greedy: argmax of a row that holds a NaN");
         return;
     }
     for (int s = 1; s < steps; ++s) {

@@ -79,7 +79,7 @@ class QwenExec {
     void expose(const std::string& name) { dec_exposed_ = dec_exposed_ || name.rfind("dec.", 0) == 0; }
     void run_decode_steps(int steps);  // Fast mode: replays the recorded decode step `steps` times (state on device)
     void set_decode_state(const int32_t* ids, const int32_t* pos);
-    void read_decode_ids(int32_t* out, int count);
+    void read_decode_ids(int32_t* out, int count, int first = 0);  // ids first .. first + count - 1 (step-major)
     // Fast mode, one sequence: true when the decode step is the single persistent launch (decode_step_persistent),
     // false when it is the recorded list of per-stage kernels. The persistent step is used when the device has at least
     // 256 CUs, the kernel covers the shape and LRM_HIP_DECODE is not "kernels" at construction.
@@ -144,7 +144,8 @@ class QwenExec {
     std::vector<uint64_t> pieces_;                 // submissions of the running forward
     hipEvent_t ev_[2] = {nullptr, nullptr};        // around the device work that last_ms() reports
     std::vector<uint32_t> dec_state_;              // the device's decode state as the host knows it; empty: not known
-    int dec_ids_ = 0;                              // ids of the last run in the device's host words
+    std::vector<uint32_t> dec_ids_;                // ids dec_id0_ .. of the runs since the state was set, as far as known
+    uint64_t dec_id0_ = 0;
     bool dec_exposed_ = false;
     bool persist_aborted_ = false;                 // the last persistent run aborted: the exchange area starts over
     uint32_t persist_wait_ = 0;                    // the wait bound the exchange header holds

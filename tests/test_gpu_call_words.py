@@ -1,5 +1,5 @@
-"""The words a call exchanges with the device (token ids on either side of the count up to which kernels carry them), and its
-command lists released before they are waited for."""
+"""The words a call exchanges with the device (token ids on either side of the count up to which kernels carry them, the
+decoded ids over many runs), and its command lists released before they are waited for."""
 import numpy as np
 import pytest
 
@@ -49,3 +49,56 @@ def test_one_shot_lists_released_before_the_wait():
         assert np.array_equal(s.read("x8"), x * 256)
     finally:
         s.close()
+
+
+def test_decode_ids_over_many_runs():
+    """decode_ids is the same however the steps are cut into runs: past 4,096 ids in all, after a run too long for the host
+    words, between runs, after a new start, and after greedy (whose first id is the prefill's)."""
+    cfg = QwenConfig(1, 1024, 16, 8, 128, 1024, 512, 1024)
+    b = HipBackend(0)
+    m = QwenModel(b, cfg, mode="fast", max_tokens=64, batch=8)
+    m.load_weights(synthetic_weights(cfg, seed=9))
+    for s in range(8):
+        m.forward(synthetic_ids(9, f"ids{s}", 5, 512), 0, logits_rows=0, seq=s)
+
+    def run(parts, look=False):
+        m.decode_set(np.arange(8, dtype=np.int32), np.full(8, 5, np.int32))
+        seen = []
+        for i, n in enumerate(parts):
+            m.decode_run(n)
+            if look:
+                seen.append(m.decode_ids(sum(parts[:i + 1]) * 8))
+        return m.decode_ids(sum(parts) * 8), seen
+    try:
+        one = run([560])[0]  # one run of 4,480 ids: read back from the device
+        many, seen = run([1, 2, 500, 40, 17], look=True)
+        assert np.array_equal(many, one) and all(np.array_equal(x, one[:x.size]) for x in seen)
+        assert np.array_equal(run([520, 40])[0], one)
+        assert np.array_equal(run([3])[0], one[:24]) and np.array_equal(m.decode_ids(8), one[:8])
+    finally:
+        m.close()
+        b.close()
+
+
+@pytest.mark.parametrize("decode", ["persistent", "kernels"])
+def test_greedy_then_decode_ids(decode, monkeypatch):
+    monkeypatch.setenv("LRM_HIP_DECODE", decode)
+    cfg = QwenConfig(1, 1024, 16, 8, 128, 3072, 512, 256)
+    b = HipBackend(0)
+    m = QwenModel(b, cfg, mode="fast", max_tokens=64)
+    m.load_weights(synthetic_weights(cfg, seed=4))
+    ids = synthetic_ids(4, "greedy", 20, 512)
+    try:
+        out = m.greedy(ids, 9)
+        assert np.array_equal(m.decode_ids(9)[1:], out[1:])
+        m.decode_run(3)  # from greedy's state
+        longer = m.greedy(ids, 12)
+        assert np.array_equal(longer[:9], out)
+        _, first = m.forward(ids, 0, logits_rows=1)
+        m.decode_set(first, 20)
+        m.decode_run(4)
+        m.decode_run(7)
+        assert first == out[0] and np.array_equal(m.decode_ids(11), longer[1:])
+    finally:
+        m.close()
+        b.close()
