@@ -316,10 +316,12 @@ __global__ __launch_bounds__(W == 1 ? 256 : 64 * W) void k_attention_mfma(
     constexpr int REGS = HD / 4;  // O registers per lane: 16 columns x HD over 64 lanes
     const uint32_t lane = threadIdx.x & 63u, wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const uint32_t col = lane & 15u, grp = lane >> 4;
-    const uint32_t group = qh / kvh, kvhead = blockIdx.y, total = rows * group, tiles = (total + 15u) / 16u;
-    const uint32_t tb = W == 1 ? blockIdx.x * 4u + wv : blockIdx.x;
+    const uint32_t group = qh / kvh, total = rows * group, tiles = (total + 15u) / 16u;
+    // the longest first; W = 1, where workgroups wait for their turn, over all KV heads (one dimension: head fastest)
+    const uint32_t kvhead = W == 1 ? blockIdx.x % kvh : blockIdx.y;
+    const uint32_t tb = W == 1 ? blockIdx.x / kvh * 4u + wv : blockIdx.x;
     if (tb >= tiles) return;
-    const uint32_t tile = tiles - 1u - tb;  // the longest first
+    const uint32_t tile = tiles - 1u - tb;
     const uint32_t raw = tile * 16u + col, idx = raw < total ? raw : total - 1u;
     const uint32_t row = idx / group, head = kvhead * group + idx % group;
     const uint32_t keys = past + row + 1u;                       // this column's
@@ -418,7 +420,7 @@ __global__ __launch_bounds__(W == 1 ? 256 : 64 * W) void k_attention_mfma(
         // A key past a column's own has weight 0, and its product is a zero of its value's sign: it leaves the chain as it is
         // while the value is finite and the chain is not -0 (a chain of products that underflow). Where a block with such
         // keys holds an infinity or a NaN, or ends at a zero, each column runs alone with those values at -0 (a product of
-        // -0 changes no chain). The look at the ends costs 512 rows of 16 heads 52.0 -> 54.1 us, 4096 rows 1310 -> 1321.
+        // -0 changes no chain). The look at the ends costs 512 rows of 16 heads 52.0 -> 54.1 us.
         const bool partial = b * 64u + 64u > first_keys;
         bool odd = false;
         if (partial) {
@@ -766,10 +768,11 @@ static void launch_attention(const float* q, const float* kc, const float* vc, f
         return;
     }
     // One wave per tile once the tiles alone give each of the chip's 1024 SIMDs one, else eight waves share a tile. 16 heads,
-    // 8 KV heads, one against eight waves: 512 rows (512 tiles) 60.6 / 52.1 us, 1024 114.6 / 143.5, 2048 443 / 421, 4096
-    // 1313 / 1486.
+    // 8 KV heads, one against eight waves: 512 rows (512 tiles) 60.1 / 54.1 us, 512 after 2048 272 / 224, 1024 113 / 148,
+    // 1536 168 / 264, 2048 243 / 433, 4096 918 / 1520. (With the tiles of one KV head before the next one's, the last head's
+    // longest began when the others' shortest ended: 1536 rows 284 us, 2048 447, slower than eight waves, 4096 1324.)
     if (tiles * kvh >= 1024)
-        hipLaunchKernelGGL((k_attention_mfma<HD, 1>), dim3(uint32_t((tiles + 3) / 4), kvh), dim3(256), 0, s, q, kc, vc, y,
+        hipLaunchKernelGGL((k_attention_mfma<HD, 1>), dim3(uint32_t((tiles + 3) / 4) * kvh), dim3(256), 0, s, q, kc, vc, y,
                            rows, q_row0, past, qh, kvh, scale);
     else
         hipLaunchKernelGGL((k_attention_mfma<HD, 8>), dim3(uint32_t(tiles), kvh), dim3(512), 0, s, q, kc, vc, y, rows,

@@ -34,7 +34,8 @@ def test_values_of_later_keys_leave_a_negative_zero(rows, qh, kvh, hd):
     assert np.array_equal(tiled.view(np.uint32), general.view(np.uint32))
 
 
-@pytest.mark.parametrize("rows,past,qh,kvh,hd", [(37, 150, 4, 2, 16), (30, 300, 16, 8, 128), (1030, 5, 64, 32, 16)])
+@pytest.mark.parametrize("rows,past,qh,kvh,hd", [(37, 150, 4, 2, 16), (30, 300, 16, 8, 128), (1030, 5, 64, 32, 16),
+                                                 (2800, 70, 6, 3, 16)])
 def test_random_denormal_values(rows, past, qh, kvh, hd):
     r = np.random.default_rng(rows + hd)
     keys = past + rows
