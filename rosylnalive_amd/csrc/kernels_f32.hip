@@ -38,14 +38,20 @@ typedef float f32x2 __attribute__((ext_vector_type(2)));
 constexpr uint32_t kNegZeroPair = 0x80008000u;
 
 // A block computes a (16 WR TM) x (16 WC TN) tile: WR x WC multiplying waves of TM x TN MFMA tiles, as many staging
-// waves. The loop runs whole groups of D tiles of KS; tiles past k multiply the padding.
-// VEC: x and w 16-byte aligned, k a multiple of 8; otherwise element loads. FULL: k a multiple of D KS, no padding.
+// waves, in groups of D tiles of KS along k.
+// VEC: x and w 16-byte aligned, k a multiple of 8; otherwise element loads. END, where k ends: FULL, with a group, no padding;
+// GROUPS, anywhere, tiles past k multiply the padding; TILES, with the tile that holds the last of k. TILES is for k up to 512
+// (32-row tiles) or 384, where a group is most of the work (padded to groups, 17 to 150 rows of k 64 took 6.4 us against 2.8,
+// of 129 10.4 against 5.0); past that, its branches cost more than the padding (1 x 64 x 504 4.4 us in groups, 4.8 in tiles;
+// 1 x 20,000 x 1000 16.0 and 24.5).
+enum class End { FULL, GROUPS, TILES };
 // Up to three weights over one x share a launch, their column tiles side by side: a decode step's q, k and v projections
 // are 64 to 128 chains' worth of blocks each, and one after another each waits its chain out on an idle chip.
-template <int WR, int WC, int TM, int TN, int KS, int D, int NB, bool VEC, bool FULL>
+template <int WR, int WC, int TM, int TN, int KS, int D, int NB, bool VEC, End END>
 __global__ __launch_bounds__(128 * WR * WC) void k_matmul_mfma(const float* __restrict__ x, MatmulGroup group,
                                                                uint32_t m, uint32_t k) {
     constexpr int BM = 16 * WR * TM, BN = 16 * WC * TN, NT = 64 * WR * WC, STEPS = KS / 4, ROW = STEPS + 4;
+    constexpr bool FULL = END == End::FULL, TILES = END == End::TILES;
     constexpr int XR = NT / (KS / 4), WRW = NT / (KS / 8);  // rows staged per pass
     constexpr int XQ = BM / XR, WQ = BN / WRW;              // 16-byte chunks per staging thread
     static_assert(XQ >= 1 && WQ >= 1 && BM % XR == 0 && BN % WRW == 0, "whole chunks");
@@ -150,18 +156,21 @@ __global__ __launch_bounds__(128 * WR * WC) void k_matmul_mfma(const float* __re
             }
             __builtin_amdgcn_sched_barrier(0);
         };
+        auto holds = [&](uint32_t k0) { return !TILES || k0 < k; };  // a tile at k0 is loaded and stored
 #pragma unroll
-        for (int d = 0; d < D; ++d) load(d, uint32_t(d) * KS);
+        for (int d = 0; d < D; ++d)
+            if (holds(uint32_t(d) * KS)) load(d, uint32_t(d) * KS);
         store(0, 0);
-        store(1, KS);
+        if (holds(KS)) store(1, KS);
         lds_barrier();
         uint32_t k0 = 0;
         do {  // (at least once: a loop that may not run lets the compiler sink the first loads past the barrier above)
 #pragma unroll
             for (int d = 0; d < D; ++d) {
-                load(d, k0 + uint32_t(d + D) * KS);  // this set's tile is in LDS
-                store((d + 2) % D, k0 + uint32_t(d + 2) * KS);
+                if (holds(k0 + uint32_t(d + D) * KS)) load(d, k0 + uint32_t(d + D) * KS);  // this set's tile is in LDS
+                if (holds(k0 + uint32_t(d + 2) * KS)) store((d + 2) % D, k0 + uint32_t(d + 2) * KS);
                 lds_barrier();
+                if (!holds(k0 + uint32_t(d + 1) * KS)) break;
             }
             k0 += D * KS;
         } while (k0 < k);
@@ -206,6 +215,7 @@ __global__ __launch_bounds__(128 * WR * WC) void k_matmul_mfma(const float* __re
                                                                              acc[a][b], 0, 0, 0);
             __builtin_amdgcn_sched_barrier(0);
             lds_barrier();
+            if (TILES && k0 + uint32_t(d + 1) * KS >= k) break;  // (with the staging waves)
         }
         k0 += D * KS;
     } while (k0 < k);
@@ -230,12 +240,18 @@ static void launch_mfma(bool vec, const float* x, const MatmulGroup& g, uint32_t
     uint32_t tiles = 0;
     for (uint32_t i = 0; i < g.count; ++i) tiles += (g.n[i] + BN - 1) / BN;
     const dim3 grid(tiles, (m + BM - 1) / BM), block(128 * WR * WC);
+    constexpr uint32_t kTilesTo = BM == 32 ? 512 : 384;
+    auto go = [&](auto kernel) { hipLaunchKernelGGL(kernel, grid, block, 0, s, x, g, m, k); };
     if (vec && k % (D * KS) == 0 && uint64_t(k) * (BM > BN / 2 ? BM : BN / 2) * 4 < (1ull << 31))
-        hipLaunchKernelGGL((k_matmul_mfma<WR, WC, TM, TN, KS, D, NB, true, true>), grid, block, 0, s, x, g, m, k);
+        go(k_matmul_mfma<WR, WC, TM, TN, KS, D, NB, true, End::FULL>);
+    else if (vec && k <= kTilesTo)
+        go(k_matmul_mfma<WR, WC, TM, TN, KS, D, NB, true, End::TILES>);
     else if (vec)
-        hipLaunchKernelGGL((k_matmul_mfma<WR, WC, TM, TN, KS, D, NB, true, false>), grid, block, 0, s, x, g, m, k);
+        go(k_matmul_mfma<WR, WC, TM, TN, KS, D, NB, true, End::GROUPS>);
+    else if (k <= kTilesTo)
+        go(k_matmul_mfma<WR, WC, TM, TN, KS, D, NB, false, End::TILES>);
     else
-        hipLaunchKernelGGL((k_matmul_mfma<WR, WC, TM, TN, KS, D, NB, false, false>), grid, block, 0, s, x, g, m, k);
+        go(k_matmul_mfma<WR, WC, TM, TN, KS, D, NB, false, End::GROUPS>);
 }
 
 // k = 0: every output is an empty chain, +0. The tile kernels read element 0 of every row, which does not exist then.
@@ -244,6 +260,41 @@ __global__ __launch_bounds__(256) void k_zero_rows(MatmulGroup group, uint32_t m
         const uint64_t n = uint64_t(m) * group.n[i], step = uint64_t(gridDim.x) * 256u;
         for (uint64_t e = uint64_t(blockIdx.x) * 256u + threadIdx.x; e < n; e += step) group.y[i][e] = 0.f;
     }
+}
+
+// Short k, where staging through registers in groups is most of the tile kernels' time: a 16 x 64 tile per block on the
+// vector ALUs, thread t column t % 64 of rows 4 (t / 64) .., K of k staged at a time.
+template <uint32_t K>
+__global__ __launch_bounds__(256) void k_matmul_short(const float* __restrict__ x, MatmulGroup group, uint32_t m, uint32_t k) {
+    __shared__ float xs[16][K];
+    __shared__ float ws[64][K + 1];
+    uint32_t part = 0, bx = blockIdx.x;
+    while (part + 1 < group.count && bx >= (group.n[part] + 63u) / 64u) bx -= (group.n[part++] + 63u) / 64u;
+    const uint16_t* __restrict__ w = group.w[part];
+    const uint32_t t = threadIdx.x, n = group.n[part], i0 = blockIdx.y * 16u, j0 = bx * 64u, col = t % 64u, r0 = t / 64u * 4u;
+    const uint32_t rows = m - i0 < 16u ? m - i0 : 16u, cols = n - j0 < 64u ? n - j0 : 64u;
+    float acc[4] = {0.f, 0.f, 0.f, 0.f};
+    for (uint32_t p0 = 0; p0 < k; p0 += K) {
+        const uint32_t ks = k - p0 < K ? k - p0 : K;
+        if (p0) __syncthreads();
+#pragma unroll
+        for (uint32_t e = t; e < 16u * K; e += 256u)
+            if (e / K < rows && e % K < ks) xs[e / K][e % K] = x[size_t(i0 + e / K) * k + p0 + e % K];
+#pragma unroll
+        for (uint32_t e = t; e < 64u * K; e += 256u)
+            if (e / K < cols && e % K < ks)
+                ws[e / K][e % K] = __uint_as_float(uint32_t(w[size_t(j0 + e / K) * k + p0 + e % K]) << 16);
+        __syncthreads();
+        for (uint32_t p = 0; p < ks; ++p) {
+            const float wv = ws[col][p];  // (columns past n, rows past m: never stored)
+#pragma unroll
+            for (uint32_t r = 0; r < 4; ++r) acc[r] = fmaf(xs[r0 + r][p], wv, acc[r]);
+        }
+    }
+    if (col >= cols) return;
+#pragma unroll
+    for (uint32_t r = 0; r < 4; ++r)
+        if (r0 + r < rows) group.y[part][size_t(i0 + r0 + r) * n + j0 + col] = acc[r];
 }
 
 void matmul_bf16w(const float* x, const MatmulGroup& g, uint32_t m, uint32_t k, hipStream_t s) {
@@ -262,6 +313,18 @@ void matmul_bf16w(const float* x, const MatmulGroup& g, uint32_t m, uint32_t k, 
         big += uint64_t((m + 63) / 64) * ((g.n[i] + 63) / 64);
         small += uint64_t((m + 31) / 32) * ((g.n[i] + 31) / 32);
     }
+    // The short kernel up to k 32, and further where the tile kernels' blocks, of few rows or columns and 60 KB and more of
+    // LDS, need many rounds of the chip. Short kernel against tile kernels, us: 17 x 1024 x 16 3.1 / 2.7, 150 x 4096 x 16 3.7 /
+    // 4.5, 150 x 20,000 x 16 7.6 / 13.2, x 33 14.9 / 21.4, 1 x 20,000 x 16 3.1 / 3.8, 1 x 100,000 x 33 7.5 / 12.8, x 64 9.6 /
+    // 10.6, x 129 25.2 / 31.4; but 17 x 1024 x 33 5.3 / 3.1.
+    const bool wide = (big + 255) / 256 * 800 < small, many = m <= 16 ? n > 65536 : !wide && small > 1024;
+    if (k <= (!many ? 32u : m <= 16 ? (vec ? 80u : 320u) : (vec ? 32u : 128u))) {
+        uint32_t tiles = 0;
+        for (uint32_t i = 0; i < g.count; ++i) tiles += (g.n[i] + 63) / 64;
+        auto go = [&](auto kernel) { hipLaunchKernelGGL(kernel, dim3(tiles, (m + 15) / 16), dim3(256), 0, s, x, g, m, k); };
+        if (k <= 16) return go(k_matmul_short<16>);
+        return k <= 32 ? go(k_matmul_short<32>) : go(k_matmul_short<64>);
+    }
     // Up to 16 rows one MFMA tile per block: an output is one chain however many columns a block has, and two waves find
     // SIMDs of their own (1 x 1024 x 1024: 5.8 us; 32-column blocks 6.0); past 16,384 columns, where the weights' stream
     // counts, 32 columns (1 x 151,936 x 1024: 79.7 us against 84.1). Above: 32 x 32 tiles, about 26 ns a tile at k 1024
@@ -271,7 +334,7 @@ void matmul_bf16w(const float* x, const MatmulGroup& g, uint32_t m, uint32_t k, 
         launch_mfma<1, 1, 1, 1, 64, 4, 4>(vec, x, g, m, k, s);
     else if (m <= 16)
         launch_mfma<1, 2, 1, 1, 64, 8, 4>(vec, x, g, m, k, s);
-    else if ((big + 255) / 256 * 800 < small)
+    else if (wide)
         launch_mfma<2, 2, 2, 2, 64, 4, 4>(vec, x, g, m, k, s);
     else
         launch_mfma<2, 2, 1, 1, 64, 8, 4>(vec, x, g, m, k, s);

@@ -1,5 +1,6 @@
-"""matmul_bf16w and its grouped forms where k ends inside the first load: k = 0 writes +0 and reads nothing (x and w are one
-element here), k = 1 .. 9 equals CpuRef F32 bit for bit; at the row and column counts of each tile form."""
+"""matmul_bf16w and its grouped forms for short k: k = 0 writes +0 and reads nothing (x and w are one element here), every
+other equals CpuRef F32 bit for bit; at the row and column counts of each tile form, and at the k where the form changes: the
+short kernel's stages (16, 32, 64) and limits, tiles that end inside a group or with it, whole groups."""
 import numpy as np
 import pytest
 
@@ -15,7 +16,7 @@ RO = TensorFlags.READ_ONLY
 
 @pytest.mark.parametrize("m,ns", [(1, (1,)), (1, (17,)), (16, (16500,)), (17, (33,)), (700, (3000,)), (3, (40, 7)),
                                   (40, (100, 33)), (1, (16, 1, 65)), (150, (64, 31, 200))])
-@pytest.mark.parametrize("k", [0, 1, 7, 8, 9])
+@pytest.mark.parametrize("k", [0, 1, 7, 8, 9, 16, 17, 32, 33, 40, 64, 65, 72, 128, 129, 200, 257, 384, 385, 392, 504, 511, 520])
 def test_matmul_short_k(m, ns, k):
     r = np.random.default_rng(m + k)
     x = r.standard_normal((m, max(k, 1)))[:, :k].astype(np.float32) if k else np.zeros((m, 0), np.float32)
@@ -37,5 +38,19 @@ def test_matmul_short_k(m, ns, k):
         for i, n in enumerate(ns):
             ref = cpuref.matmul_bf16w(x, ws[i]) if k else np.zeros((m, n), np.float32)
             assert got[f"y{i}"].tobytes() == ref.tobytes(), i
+    finally:
+        s.close()
+
+
+@pytest.mark.parametrize("m,n,k", [(1, 65537, 64), (3, 65540, 80), (1, 65537, 88), (2, 65600, 319), (1, 65537, 321),
+                                   (40, 20000, 32), (40, 20000, 40), (33, 20001, 33), (40, 20000, 127), (40, 20000, 130)])
+def test_matmul_short_k_of_many_tiles(m, n, k):
+    r = np.random.default_rng(m + k)
+    x = r.standard_normal((m, k)).astype(np.float32)
+    w = cpuref.bf16_narrow(r.standard_normal((n, k)).astype(np.float32))
+    s = Session({"x": (F32, x.shape, RO, x), "w": (BF16, w.shape, RO, w), "y": (F32, (m, n), 0, None)})
+    try:
+        y = s.run("matmul_bf16w", ["y"], x="x", w="w", y="y", m=m, n=n, k=k)["y"]
+        assert y.tobytes() == cpuref.matmul_bf16w(x, w).tobytes()
     finally:
         s.close()
