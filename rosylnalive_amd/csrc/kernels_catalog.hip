@@ -239,10 +239,10 @@ __global__ __launch_bounds__(256) void k_add_rmsnorm_rows(const float* a, const 
 
 // ---------------------------------------------------------------- 11 argmax_rows
 // The lowest index of the row maximum by '>' (+0 and -0 tie); a row holding a NaN gives 0xFFFFFFFF.
-// 1024 threads with four loads in flight each: a row's time is its loads' latency (4,096 columns: 7.1 us with 256 threads,
-// one load at a time).
-constexpr uint32_t AM_T = 1024;
-__global__ __launch_bounds__(1024) void k_argmax_rows(const float* x, uint32_t* y, uint32_t rows, uint32_t cols) {
+// A row's time is its loads' latency, so AM_T threads with four loads in flight each; many rows take turns on the chip, and a
+// workgroup of 1024 threads costs then what 16 of 64 do (l_argmax).
+template <uint32_t AM_T>
+__global__ __launch_bounds__(AM_T) void k_argmax_rows(const float* x, uint32_t* y, uint32_t rows, uint32_t cols) {
     __shared__ float sv[AM_T];
     __shared__ uint32_t si[AM_T];
     __shared__ int snan;
@@ -405,7 +405,19 @@ static void l_copy_rows(const PreparedDispatch& pd, void* const* p, hipStream_t 
                        pd.words[4], pd.words[5], pd.words[6], pd.words[7], pd.words[8]);
 }
 static void l_argmax(const PreparedDispatch& pd, void* const* p, hipStream_t s) {
-    hipLaunchKernelGGL(k_argmax_rows, phys(pd), dim3(AM_T), 0, s, (const float*)p[0], (uint32_t*)p[1], pd.words[3], pd.words[4]);
+    // Rows x columns, us with 64 / 256 / 1024 threads: 1 x 512 2.9 / 3.1 / 3.4, 4096 x 512 4.6 / 7.1 / 23, 1 x 2048 4.5 / 3.2 /
+    // 3.6, 1 x 4096 6.6 / 3.9 / 3.6, 512 x 4096 7.3 / 4.8 / 4.8, 4096 x 4096 13 / 15 / 28, 512 x 16,384 21 / 9.1 / 7.0, 1000 x
+    // 16,384 31 / 14 / 15, 512 x 151,936 350 / 110 / 51 (256 threads with one load at a time: 4096 x 512 6.6, 1 x 4096 5.0).
+    const uint32_t rows = pd.words[3], cols = pd.words[4];
+    auto go = [&](auto kernel, uint32_t threads) {
+        hipLaunchKernelGGL(kernel, phys(pd), dim3(threads), 0, s, (const float*)p[0], (uint32_t*)p[1], rows, cols);
+    };
+    if (cols <= 512)
+        go(k_argmax_rows<64>, 64);
+    else if (cols > 32768 || (cols >= 4096 && rows <= 512))
+        go(k_argmax_rows<1024>, 1024);
+    else
+        go(k_argmax_rows<256>, 256);
 }
 static void l_matmul(const PreparedDispatch& pd, void* const* p, hipStream_t s) {
     const f32k::MatmulGroup g{{(const uint16_t*)p[1], nullptr, nullptr}, {(float*)p[2], nullptr, nullptr}, {pd.words[5], 0, 0}, 1};
