@@ -810,15 +810,25 @@ __global__ __launch_bounds__(HD < 64 ? 64 : HD) void k_row_combine(RowWorkspace 
 }
 
 template <int HD>
-static void launch_attention(const float* q, const float* kc, const float* vc, float* y, uint32_t rows, uint32_t q_row0,
+static bool launch_attention(const float* q, const float* kc, const float* vc, float* y, uint32_t rows, uint32_t q_row0,
                              uint32_t past, uint32_t qh, uint32_t kvh, float scale, void* workspace,
                              hipStream_t s) {
     const uint64_t tiles = (uint64_t(rows) * (qh / kvh) + 15) / 16;
     const uint32_t group = qh / kvh, nb = past / 64u + 1u;
     // (three launches against one: at 64 and 128 dimensions they win from the first key, 63 keys 10 us against 14; below,
     // where a block is little work, from eight blocks on)
-    if (workspace && rows == 1 && (HD >= 64 || nb >= 8) && (group == 1 || group == 2 || group == 4) && uint64_t(64) * kvh * HD < (1ull << 30) &&
-        RowWorkspace::bytes(qh, nb, HD) <= kWorkspaceBytes) {
+    const bool spread = workspace && rows == 1 && (HD >= 64 || nb >= 8) && (group == 1 || group == 2 || group == 4) &&
+                        uint64_t(64) * kvh * HD < (1ull << 30) && RowWorkspace::bytes(qh, nb, HD) <= kWorkspaceBytes;
+    // Of a few keys a tile's loads and exchanges of 64 are most of its time, and the general kernel, a workgroup per row and
+    // head, is done before. 16 heads, general kernel against this file's, us: 1 key of 16 dimensions 3.2 / 5.2, 9 keys 4.9 / 5.3,
+    // 12 keys 5.5 / 5.3; 1 row at 9 keys of 64, over the chip, 7.7 / 9.4, at 16 9.5 / 9.6; 9 rows of 128 12.7 / 14.8, 12 rows
+    // 14.1 / 14.8, 16 rows 15.3 / 14.9; but 1 row at 8 keys of 128, over the chip, 12.2 / 10.1. Many rows and heads take longer
+    // than a tile each on its CU (512 heads, 8 rows of 16: 6.6 / 5.7), but not than the tiles' second turn (9 rows of 128: 17.9
+    // / 29.6).
+    const uint32_t few = HD == 64 && spread ? 13 : HD == 128 ? (spread ? 0 : 12) : 10;
+    const bool second = HD >= 32 && tiles * kvh > 256 && tiles * kvh <= 384;
+    if (uint64_t(past) + rows <= few && (uint64_t(rows) * qh <= 3072 || second)) return false;
+    if (spread) {
         const RowWorkspace ws(static_cast<float*>(workspace), qh, nb);
         auto go = [&](auto scores, auto values, uint32_t threads) {
             hipLaunchKernelGGL(scores, dim3(nb, kvh), dim3(256), 0, s, q, kc, ws, q_row0, past, qh, kvh, scale);
@@ -828,7 +838,7 @@ static void launch_attention(const float* q, const float* kc, const float* vc, f
         if (group == 2) go(k_row_scores<HD, 2>, k_row_values<HD, 2>, 2 * HD);
         if (group == 4) go(k_row_scores<HD, 4>, k_row_values<HD, 4>, 4 * HD);
         hipLaunchKernelGGL(k_row_combine<HD>, dim3(qh), dim3(HD < 64 ? 64 : HD), 0, s, ws, y, q_row0, qh, nb);
-        return;
+        return true;
     }
     // One wave per tile once the tiles alone give each of the chip's 1024 SIMDs one, else eight waves share a tile. 16 heads,
     // 8 KV heads, one against eight waves: 512 rows (512 tiles) 60.1 / 54.1 us, 512 after 2048 272 / 224, 1024 113 / 148,
@@ -840,16 +850,17 @@ static void launch_attention(const float* q, const float* kc, const float* vc, f
     else
         hipLaunchKernelGGL((k_attention_mfma<HD, 8>), dim3(uint32_t(tiles), kvh), dim3(512), 0, s, q, kc, vc, y, rows,
                            q_row0, past, qh, kvh, scale);
+    return true;
 }
 
 bool attention(const float* q, const float* kc, const float* vc, float* y, uint32_t rows, uint32_t q_row0, uint32_t past,
                uint32_t qh, uint32_t kvh, uint32_t hd, float scale, void* workspace, hipStream_t s) {
     if (!aligned16(q) || !aligned16(kc) || !aligned16(vc) || uint64_t(rows) * (qh / kvh) > 0x7FFFFFFFull) return false;
     switch (hd) {
-        case 16: launch_attention<16>(q, kc, vc, y, rows, q_row0, past, qh, kvh, scale, workspace, s); return true;
-        case 32: launch_attention<32>(q, kc, vc, y, rows, q_row0, past, qh, kvh, scale, workspace, s); return true;
-        case 64: launch_attention<64>(q, kc, vc, y, rows, q_row0, past, qh, kvh, scale, workspace, s); return true;
-        case 128: launch_attention<128>(q, kc, vc, y, rows, q_row0, past, qh, kvh, scale, workspace, s); return true;
+        case 16: return launch_attention<16>(q, kc, vc, y, rows, q_row0, past, qh, kvh, scale, workspace, s);
+        case 32: return launch_attention<32>(q, kc, vc, y, rows, q_row0, past, qh, kvh, scale, workspace, s);
+        case 64: return launch_attention<64>(q, kc, vc, y, rows, q_row0, past, qh, kvh, scale, workspace, s);
+        case 128: return launch_attention<128>(q, kc, vc, y, rows, q_row0, past, qh, kvh, scale, workspace, s);
         default: return false;
     }
 }

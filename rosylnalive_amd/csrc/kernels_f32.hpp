@@ -17,7 +17,8 @@ struct MatmulGroup {
 };
 void matmul_bf16w(const float* x, const MatmulGroup& group, uint32_t m, uint32_t k, hipStream_t s);
 
-// attention_gqa_causal on the matrix cores; false (nothing launched) when the shape or an alignment is not covered. A
+// attention_gqa_causal on the matrix cores; false (nothing launched) where the general kernel takes the call: a shape or an
+// alignment that is not covered, or too few keys to be worth it. A
 // decode row spreads over the chip when `workspace` (kWorkspaceBytes, written by each call, its contents not kept; null:
 // none) holds its blocks: of the 0.6B's 16 heads, up to 21,500 keys.
 constexpr uint64_t kWorkspaceBytes = uint64_t(4) << 20;

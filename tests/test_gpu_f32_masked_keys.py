@@ -43,3 +43,15 @@ def test_random_denormal_values(rows, past, qh, kvh, hd):
     v = (r.integers(-2, 3, (keys, kvh * hd)) * np.float64(ULP)).astype(np.float32)
     tiled, general = _attention(q, k, v, qh, kvh, hd, past, 0), _attention(q, k, v, qh, kvh, hd, past, 1)
     assert np.array_equal(tiled.view(np.uint32), general.view(np.uint32))
+
+
+@pytest.mark.parametrize("hd", [16, 32, 64, 128])
+@pytest.mark.parametrize("rows,past,qh,kvh", [(1, 0, 4, 2), (1, 9, 16, 8), (1, 10, 16, 8), (1, 12, 6, 2), (1, 13, 4, 1),
+                                              (3, 7, 16, 8), (3, 8, 16, 8), (12, 0, 16, 8), (13, 0, 4, 4), (9, 0, 512, 128),
+                                              (6, 0, 512, 256)])
+def test_few_keys(rows, past, qh, kvh, hd):
+    """Either side of the counts up to which the general kernel takes aligned tensors too."""
+    r = np.random.default_rng(rows + past + hd)
+    q, k, v = (r.standard_normal((n, h * hd)).astype(np.float32) for n, h in ((rows, qh), (past + rows, kvh), (past + rows, kvh)))
+    tiled, general = _attention(q, k, v, qh, kvh, hd, past, 0), _attention(q, k, v, qh, kvh, hd, past, 1)
+    assert np.array_equal(tiled.view(np.uint32), general.view(np.uint32))
