@@ -2232,18 +2232,21 @@ static bool two_per_cu(const dim3& g) {
 // it multiplies) of them takes 0.63 / 0.5 of a round of the largest: the fewest such units win, the larger tile on a tie.
 // Four layers, device time, against 128 rows up to 64 rows and 64 from there to 256 tiles: 0.6B shape at 37 rows 284 -> 195
 // us, 100 253 -> 207, 256 267 -> 230; 1.7B at 37 412 -> 314, 100 386 -> 339. The sums' order does not depend on the tile.
-static int small_tile(uint64_t full, uint64_t rows64, uint64_t half) {
+// price64: the 64-row form's where it is another (per cent of the largest's round).
+static int small_tile(uint64_t full, uint64_t rows64, uint64_t half, uint64_t price64 = 63) {
     auto rounds = [](uint64_t tiles) { return (tiles + 255) / 256; };
-    const uint64_t a = rounds(full) * 100, b = rounds(rows64) * 63, c = half ? rounds(half) * 50 : ~uint64_t(0);
+    const uint64_t a = rounds(full) * 100, b = rounds(rows64) * price64, c = half ? rounds(half) * 50 : ~uint64_t(0);
     return a <= b && a <= c ? 0 : b <= c ? 1 : 2;
 }
 static uint64_t tiles_of(uint64_t m, uint64_t rows, uint64_t n, uint64_t cols) {
     return ((m + rows - 1) / rows) * ((n + cols - 1) / cols);
 }
-// gemm_qkv_rope's tile, one head wide: 128 rows on the direct-to-LDS loop (-1), or the register loop's 128 (0) or 64 (1)
+// gemm_qkv_rope's tile, one head wide: 128 rows on the direct-to-LDS loop (-1), or the register loop's 128 (0) or 64 (1), whose
+// round costs more here, for the heads' epilogue (k 1024: three rounds of 64 rows 29.4 us at 48 heads and 700 rows, two of 128
+// 28.0).
 static int qkv_tile(uint32_t m, uint32_t heads) {
     if (two_per_cu(dim3(heads, (m + 127) / 128))) return -1;
-    return small_tile(tiles_of(m, 128, heads, 1), tiles_of(m, 64, heads, 1), 0);
+    return small_tile(tiles_of(m, 128, heads, 1), tiles_of(m, 64, heads, 1), 0, 67);
 }
 static dim3 qkv_grid(uint32_t m, uint32_t heads) {
     return dim3(heads, qkv_tile(m, heads) == 1 ? (m + 63) / 64 : (m + 127) / 128);
@@ -2634,14 +2637,18 @@ static bool resid_split_skinny(uint32_t m, uint32_t k, uint32_t splits) {
     return m <= 16 && (k / splits) % (kSkWaves * 128) == 0;
 }
 // its tile: 128 x 64 on the direct-to-LDS loop (-1; four layers at 777 rows of the 0.6B shape, 448 tiles: 411 -> 399 us) or
-// the register loop's 128 x 64 (0), 64 x 64 (1) or 64 x 32 (2)
-static int resid_tile(uint32_t m, uint32_t n, uint32_t splits) {
+// the register loop's 128 x 64 (0), 64 x 64 (1) or 64 x 32 (2). Here the direct loop gains less per tile and loses a partly
+// filled round past the first sooner: k 1024 per split, 384 tiles 14.6 us against 16.1, 768 23.6 / 22.9, 832 26.6 / 27.6, 1152
+// 34.4 / 33.4, 1664 46.1 / 44.7. Splits of under 512 k are bound by their partials' stores, which two rounds of 64 rows spread
+// better than one of 128 (513 x 1000 of 256 k in two splits 5.5 us against 6.0).
+static int resid_tile(uint32_t m, uint32_t n, uint32_t k, uint32_t splits) {
     const uint64_t full = tiles_of(m, 128, n, 64) * splits;
-    if (mostly_full(full)) return -1;
-    return small_tile(full, tiles_of(m, 64, n, 64) * splits, tiles_of(m, 64, n, 32) * splits);
+    if (full % 512 == 0 || (full <= 512 && mostly_full(full)) || (full <= 1024 && full >= 832)) return -1;
+    const uint64_t rows64 = tiles_of(m, 64, n, 64) * splits;
+    return small_tile(full, rows64, tiles_of(m, 64, n, 32) * splits, k / splits < 512 && rows64 > 256 ? 49 : 63);
 }
-static dim3 resid_grid(uint32_t m, uint32_t n, uint32_t splits) {
-    const int t = resid_tile(m, n, splits);
+static dim3 resid_grid(uint32_t m, uint32_t n, uint32_t k, uint32_t splits) {
+    const int t = resid_tile(m, n, k, splits);
     return dim3(t == 2 ? (n + 31) / 32 : (n + 63) / 64, t > 0 ? (m + 63) / 64 : (m + 127) / 128, splits);
 }
 static void l_gemm_resid_split(const PreparedDispatch& pd, void* const* p, hipStream_t s) {
@@ -2656,8 +2663,8 @@ static void l_gemm_resid_split(const PreparedDispatch& pd, void* const* p, hipSt
     a.y32 = (float*)p[2];
     a.ksplit = int(w[6] / w[7]);
     a.ascale = a_unscale(w[8]);
-    const dim3 grid = resid_grid(w[4], w[5], w[7]);
-    switch (resid_tile(w[4], w[5], w[7])) {
+    const dim3 grid = resid_grid(w[4], w[5], w[6], w[7]);
+    switch (resid_tile(w[4], w[5], w[6], w[7])) {
         case -1: hipLaunchKernelGGL((k_gemm<EPI_PART, 64, true>), grid, dim3(256), 0, s, a); break;
         case 0: hipLaunchKernelGGL((k_gemm<EPI_PART, 64, false>), grid, dim3(256), 0, s, a); break;
         case 1: hipLaunchKernelGGL((k_gemm<EPI_PART, 64, false, 64>), grid, dim3(256), 0, s, a); break;
@@ -3092,7 +3099,7 @@ std::vector<KernelSpec> fast_catalog() {
     c.push_back({"gemm_residual_split", "fast", {256, 1, 1}, false,
                  [](const uint32_t* w) {
                      if (resid_split_skinny(w[4], w[6], w[7])) return Grid3{(int64_t(w[5]) + 15) / 16, w[7], 1};
-                     const dim3 g = resid_grid(w[4], w[5], w[7]);
+                     const dim3 g = resid_grid(w[4], w[5], w[6], w[7]);
                      return Grid3{g.x, g.y, g.z};
                  },
                  {TOK_R("a", DT(F16)), TOK_R("w", DT(F16)), TOK_W("partials", DT(F32)), U32F("m"), U32F("n"), U32F("k"),
