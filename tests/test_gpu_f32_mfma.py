@@ -1,12 +1,12 @@
 """The float32 contractions on the matrix cores (kernels_f32.hip) at the sizes where their tiles end.
 
-- matmul_bf16w: every dispatch (one or two rows, 16 x 64, 32 x 32 and 64 x 64 tiles; 16-byte and element loads) at
+- matmul_bf16w: every tile (16 x 16 and 16 x 32 up to 16 rows, 32 x 32 and 64 x 64 above; 16-byte and element loads) at
   remainders of rows, columns and k equals CpuRef F32 bit for bit, rows whose products underflow to -0 included (the
   padding past k must keep a chain's -0).
 - attention_gqa_causal: the matrix-core kernel (16-byte aligned tensors, head_dim 16, 32, 64, 128) equals the general
   kernel, which the same tensors one float off their alignment take, bit for bit: one wave per tile and eight, tiles that
-  end inside a row's heads, block edges, the single query row's three launches (up to and past their workspace), and an infinity or NaN among the
-  values of keys past a query's own, which only the queries that own them may see.
+  end inside a row's heads, block edges, the single query row's three launches up to the end of their workspace, and an
+  infinity or NaN among the values of keys past a query's own, which only the queries that own them may see.
 """
 import numpy as np
 import pytest
