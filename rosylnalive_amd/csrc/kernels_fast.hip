@@ -242,7 +242,7 @@ struct GemmStampEnd {  // the epilogue's end, at whichever return the lane leave
 
 // Two main loops, chosen by the launcher: DMA (a grid of at least two blocks per CU) moves tiles from memory
 // straight into two LDS stages, the two blocks on a CU hiding each other's load latency; otherwise (one block per CU)
-// tiles go through two register sets into two padded LDS buffers with every load two k steps ahead.
+// tiles go through two register sets into two LDS buffers with every load two k steps ahead.
 template <int EPI, int BN, bool DMA, int BM = GBM>
 __global__ __launch_bounds__(256, 2) void k_gemm(GemmArgs p) {
     static_assert(BN == 128 || (BN == 64 && EPI != EPI_QKV && (EPI != EPI_SWIGLU || BM == 64)) ||
@@ -2217,11 +2217,11 @@ static GemmArgs gemm_base(void* const* p, uint32_t m, uint32_t n, uint32_t k) {
     return a;
 }
 
-// The GEMM's direct-to-LDS loop needs two blocks on every CU (MI355X: 256 CUs, two 64 KiB blocks each) for most of the
-// launch: rounds of 512 tiles at least three quarters full, or so many (4) that a partial last one hardly counts. In an
-// emptier round a CU holds one block, which the register-pipelined loop (loads two k steps ahead) serves better (measured:
-// the 768-tile SwiGLU GEMM of a 2048-token prefill, 42 against 44 us). Four layers, device time, against whole rounds only:
-// 0.6B shape at 1000 rows (384 SwiGLU tiles) 437 -> 423 us, 1800 (480 q|k|v tiles) 625 -> 609; 1.7B at 600 641 -> 625.
+// The GEMM's direct-to-LDS loop wants two blocks on every CU (MI355X: 256 CUs, two 64 KiB blocks each) for most of the
+// launch: rounds of 512 tiles at least three quarters full, or so many (4) that a partial last one hardly counts (gate / up
+// at k 1024: 384 tiles 20.2 us, the register loop's 128 rows 23.6; 768 32.8 / 36.0). Emptier rounds go to the register loop
+// (loads two k steps ahead), whose smaller tiles reach more CUs. Four layers, device time, against whole rounds only: 0.6B
+// shape at 1000 rows (384 SwiGLU tiles) 437 -> 423 us, 1800 (480 q|k|v tiles) 625 -> 609; 1.7B at 600 641 -> 625.
 static bool mostly_full(uint64_t tiles) { return tiles * 4 >= (tiles + 511) / 512 * (512 * 3); }
 static bool two_per_cu(const dim3& g) {
     const uint64_t tiles = uint64_t(g.x) * g.y;
@@ -2346,7 +2346,9 @@ static void l_gemm_swiglu(const PreparedDispatch& pd, void* const* p, hipStream_
         hipLaunchKernelGGL((k_gemm<EPI_SWIGLU, 128, false>), grid, dim3(256), 0, s, a);
 }
 
-// gemm_f32's tile: 128 columns, 64 in the register loop's smallest form
+// gemm_f32's tile: 128 columns, 64 in the register loop's smallest form. The direct-to-LDS loop on whole rounds only: its
+// calls are mostly lm_heads of one row tile, which partial rounds of it lose (151,936 x 1024, 1187 tiles: 64 rows 74.6 us, 81.5
+// on the direct loop; x 2048 145 / 170), while several row tiles would gain (12,288 x 1024 at 512 rows, 384 tiles: 22.6 / 20.7).
 static bool f32_dma(uint32_t m, uint32_t n) {
     const uint64_t tiles = tiles_of(m, 128, n, 128);
     return tiles >= 512 && (tiles % 512 == 0 || tiles >= 4 * 512);

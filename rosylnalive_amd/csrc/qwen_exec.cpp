@@ -792,8 +792,10 @@ static bool add_norm_width(uint32_t n) { return n == 256 || n == 512 || n == 102
 static uint32_t resid_splits(uint32_t m, uint32_t n, uint32_t k, uint32_t max_tokens) {
     if (!add_norm_width(n)) return 1;
     const uint64_t tiles = uint64_t((n + 63) / 64) * ((m + 127) / 128);
-    // up to 512 rows the GEMM runs 64-row tiles, and two splits then fill the CUs with half the partials for
-    // residual_add_norm to add (512-token forward: 2.27 -> 2.24 ms against four splits of 128-row tiles)
+    // Two up to 512 rows: half the partials for residual_add_norm to add. Device time of four layers with two / four splits:
+    // 0.6B shape at 37 rows 195 / 186 us, 200 230 / 232, 512 280 / 290, 777 370 / 377; 1.7B at 37 312 / 287, 300 428 / 441, 512
+    // 500 / 522, 777 668 / 696. (Under 200 rows four would be the faster; the count decides the order of every row's sums, so
+    // it stays.)
     const uint32_t smax = m <= 512 ? 2 : 4;
     uint32_t s = 1;
     while (s < smax && tiles * s < 512 && 2 * s * m <= 2 * max_tokens && k % (128 * s) == 0) s *= 2;
